@@ -81,14 +81,8 @@ __device__ inline void march2d(const T* __restrict__ pop, T* __restrict__ pop_sw
 #pragma unroll
       for (int k = 0; k <= 2 * R; k++) sl[k] = (j - 2 * R + k) % NS;
       const int cx = R + tid;
-      T gx = 0, gy = 0, gz = 0;
-#pragma unroll
-      for (int e = 0; e < ES::QE; e++) {
-        const T v = lds[sl[R + ES::ey[e]]][cx + ES::ex[e]];
-        const T w = T(ES::w[e]);
-        if (ES::ex[e] != 0) gx += T(ES::ex[e]) * w * v;
-        if (ES::ey[e] != 0) gy += T(ES::ey[e]) * w * v;
-      }
+      T gx, gy, gz;
+      iso_grad<ES>([&](int e) { return lds[sl[R + ES::ey[e]]][cx + ES::ex[e]]; }, gx, gy, gz);
       const T lpsi = lds[sl[R]][cx];
       T fo[Q], u[3];
       collide<S, T, SHIFT, 0>(fh[0], dnh[0], gx, gy, gz, lpsi, P, fo, u);
@@ -217,14 +211,8 @@ k_batched_tile(const T* __restrict__ pop_all, T* __restrict__ swap_all,
     }
     __syncthreads();
     if (x < d.L0 && y < d.L1) {
-      T gx = 0, gy = 0;
-#pragma unroll
-      for (int e = 0; e < ES::QE; e++) {
-        const T v = lds[ty + R + ES::ey[e]][tx + R + ES::ex[e]];
-        const T wgt = T(ES::w[e]);
-        if (ES::ex[e] != 0) gx += T(ES::ex[e]) * wgt * v;
-        if (ES::ey[e] != 0) gy += T(ES::ey[e]) * wgt * v;
-      }
+      T gx, gy, gz;
+      iso_grad<ES>([&](int e) { return lds[ty + R + ES::ey[e]][tx + R + ES::ex[e]]; }, gx, gy, gz);
       T fo[Q], u[3];
       collide<S, T, SHIFT, 0>(f, s, gx, gy, T(0), lds[ty + R][tx + R], P, fo, u);
       if constexpr (PULL) local_store<S, T>(swap_all + d.pop_off, geo, x, y, 0, fo);
@@ -325,14 +313,8 @@ __device__ __forceinline__ void tile2_body(
     const int sidx = tid + k * NT;
     const int lx = sidx % SH::LW, ly = sidx / SH::LW;
     if (sidx < SH::NL && lx >= 1 && lx < SH::LW - 1 && ly >= 1 && ly < SH::LH - 1) {
-      T gx = 0, gy = 0;
-#pragma unroll
-      for (int e = 0; e < ES::QE; e++) {
-        const T v = psi0[ly + ES::ey[e]][lx + ES::ex[e]];
-        const T wgt = T(ES::w[e]);
-        if (ES::ex[e] != 0) gx += T(ES::ex[e]) * wgt * v;
-        if (ES::ey[e] != 0) gy += T(ES::ey[e]) * wgt * v;
-      }
+      T gx, gy, gz;
+      iso_grad<ES>([&](int e) { return psi0[ly + ES::ey[e]][lx + ES::ex[e]]; }, gx, gy, gz);
       T fo[Q], u[3];
       collide<S, T, SHIFT, 0>(f0[k], s0[k], gx, gy, T(0), psi0[ly][lx], P, fo, u);
       const int c = (ly - 1) * SH::CW + (lx - 1);
@@ -360,14 +342,8 @@ __device__ __forceinline__ void tile2_body(
     T s = 0;
 #pragma unroll
     for (int q = 0; q < Q; q++) s += f[q];
-    T gx = 0, gy = 0;
-#pragma unroll
-    for (int e = 0; e < ES::QE; e++) {
-      const T v = psi1[ty + 1 + ES::ey[e]][tx + 1 + ES::ex[e]];
-      const T wgt = T(ES::w[e]);
-      if (ES::ex[e] != 0) gx += T(ES::ex[e]) * wgt * v;
-      if (ES::ey[e] != 0) gy += T(ES::ey[e]) * wgt * v;
-    }
+    T gx, gy, gz;
+    iso_grad<ES>([&](int e) { return psi1[ty + 1 + ES::ey[e]][tx + 1 + ES::ex[e]]; }, gx, gy, gz);
     T fo[Q], u[3];
     collide<S, T, SHIFT, 0>(f, s, gx, gy, T(0), psi1[ty + 1][tx + 1], P, fo, u);
     if (wsh) {

@@ -190,6 +190,37 @@ struct Acc {
   __device__ __forceinline__ T get() const { return any ? v : T(0); }
 };
 
+// xi_q . v, the zero components left out.
+template <class S, class T>
+__device__ __forceinline__ T xi_dot(int q, T vx, T vy, T vz) {
+  const int cx = S::cx[q], cy = S::cy[q], cz = S::cz[q];
+  T a = cx ? (cx > 0 ? vx : -vx) : cy ? (cy > 0 ? vy : -vy) : (cz > 0 ? vz : -vz);
+  if (cx && cy) a = cy > 0 ? a + vy : a - vy;
+  if ((cx || cy) && cz) a = cz > 0 ? a + vz : a - vz;
+  return a;
+}
+
+// Isotropic gradient sum_e w_e e psi(x + e): `at(e)` is psi at stencil vector
+// e; w_e psi is formed once and serves every component (e in {-2 .. 2}, so
+// the products with it are exact).
+template <class ES, class T, class At>
+__device__ __forceinline__ void iso_grad(At at, T& gx, T& gy, T& gz) {
+  gx = gy = gz = T(0);
+  auto acc = [](T& g, int c, T wv) {
+    if (c == 1) g += wv;
+    if (c == -1) g -= wv;
+    if (c == 2) g = fma(T(2), wv, g);
+    if (c == -2) g = fma(T(-2), wv, g);
+  };
+#pragma unroll
+  for (int e = 0; e < ES::QE; e++) {
+    const T wv = T(ES::w[e]) * at(e);
+    acc(gx, ES::ex[e], wv);
+    acc(gy, ES::ey[e], wv);
+    acc(gz, ES::ez[e], wv);
+  }
+}
+
 // True when moment k of some forcing basis vector is non-zero (Mp v_b).
 template <class S>
 __device__ constexpr bool mpv_row_nz(int k) {
@@ -279,16 +310,24 @@ __device__ inline void collide(const T (&f)[S::Q], T dn, T gx, T gy, T gz,
     const T lux = u0x + Fx / n / om, luy = u0y + Fy / n / om;
     const T luz = S::D == 3 ? u0z + Fz / n / om : T(0);
     const T uu = lux * lux + luy * luy + luz * luz;
-    T px = 0, py = 0, pz = 0;
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-      const T xu = S::cx[q] * lux + S::cy[q] * luy + S::cz[q] * luz;
-      T e = T(1);
-      e += xu * T(kCM2) + T(0.5) * xu * xu * T(kCM4);
-      e += T(-0.5) * uu * T(kCM2);
+    const T eu = T(-0.5) * uu * T(kCM2);
+    auto relax = [&](int q, T e) {
       T feq = e * n * T(S::w[q]);
       if (SHIFT) feq -= T(S::w[q]) * P.rho0;
       fo[q] = f[q] * (T(1) - om) + feq * om;
+    };
+    relax(0, T(1) + eu);
+#pragma unroll
+    for (int p = 0; p < S::NPAIR; p++) {
+      const int q = S::PairQ[p], o = S::opp[q];
+      const T xu = xi_dot<S>(q, lux, luy, luz);
+      const T e1 = xu * T(kCM2), e2 = T(0.5) * xu * xu * T(kCM4);
+      relax(q, T(1) + (e1 + e2) + eu);
+      relax(o, T(1) + (e2 - e1) + eu);
+    }
+    T px = 0, py = 0, pz = 0;
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
       if (S::cx[q] == 1) px += fo[q];
       if (S::cx[q] == -1) px -= fo[q];
       if (S::cy[q] == 1) py += fo[q];
@@ -317,14 +356,24 @@ __device__ inline void collide(const T (&f)[S::Q], T dn, T gx, T gy, T gz,
     // n-part of f_eq without the shift: SHIFT subtracts w*rho0 from f_eq,
     // i.e. uses dn in place of n for the constant term.
     const T n0 = SHIFT ? dn : n;
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-      const T xu = S::cx[q] * ux + S::cy[q] * uy + S::cz[q] * uz;
-      const T xF = S::cx[q] * Fx + S::cy[q] * Fy + S::cz[q] * Fz;
+    // opposite velocities share xi.u, xi.F and their products: those of -xi
+    // are the same numbers with the odd terms negated
+    const T cu = T(0.5 * kCM2) * uu, cF = T(kCM2) * Fu;
+    auto relax = [&](int q, T se, T sg) {
       const T w = T(S::w[q]);
-      const T feq = w * (n0 + n * (T(kCM2) * xu + T(0.5 * kCM4) * xu * xu - T(0.5 * kCM2) * uu));
-      const T fg = w * (T(kCM2) * xF + T(kCM4) * xF * xu - T(kCM2) * Fu);
+      const T feq = w * (n0 + n * (se - cu));
+      const T fg = w * (sg - cF);
       fo[q] = c_f * f[q] + om * feq + c_g * fg;
+    };
+    relax(0, T(0), T(0));
+#pragma unroll
+    for (int p = 0; p < S::NPAIR; p++) {
+      const int q = S::PairQ[p], o = S::opp[q];
+      const T xu = xi_dot<S>(q, ux, uy, uz), xF = xi_dot<S>(q, Fx, Fy, Fz);
+      const T e1 = T(kCM2) * xu, e2 = T(0.5 * kCM4) * xu * xu;
+      const T g1 = T(kCM2) * xF, g2 = T(kCM4) * xF * xu;
+      relax(q, e1 + e2, g1 + g2);
+      relax(o, e2 - e1, g2 - g1);
     }
     // COLL 4: BGK with Guo forcing, then the isotropy filter (D2Q9, FP64)
     if constexpr (COLL == 4) iso_filter<S, T>(fo);
@@ -734,17 +783,14 @@ __device__ __forceinline__ void fused_body(const T* __restrict__ pop, T* __restr
       for (int q = 0; q < Q; q++) s += f[q];
       const int cy = D == 3 ? R + iy : 0;
       const int cx = R + ix;
-      T gx = 0, gy = 0, gz = 0;
-#pragma unroll
-      for (int e = 0; e < ES::QE; e++) {
-        const int em = D == 3 ? ES::ez[e] : ES::ey[e];
-        const int ey = D == 3 ? ES::ey[e] : 0;
-        const T v = lds[(j - R + em) % NS][cy + ey][cx + ES::ex[e]];
-        const T w = T(ES::w[e]);
-        if (ES::ex[e] != 0) gx += T(ES::ex[e]) * w * v;
-        if (ES::ey[e] != 0) gy += T(ES::ey[e]) * w * v;
-        if (ES::ez[e] != 0) gz += T(ES::ez[e]) * w * v;
-      }
+      T gx, gy, gz;
+      iso_grad<ES>(
+          [&](int e) {
+            const int em = D == 3 ? ES::ez[e] : ES::ey[e];
+            const int ey = D == 3 ? ES::ey[e] : 0;
+            return lds[(j - R + em) % NS][cy + ey][cx + ES::ex[e]];
+          },
+          gx, gy, gz);
       const T lpsi = lds[(j - R) % NS][cy][cx];
       T fo[Q], u[3];
       collide<S, T, SHIFT, COLL>(f, s, gx, gy, gz, lpsi, P, fo, u);
@@ -828,17 +874,14 @@ __device__ __forceinline__ void fused_body(const T* __restrict__ pop, T* __restr
       for (int k = 0; k <= 2 * R; k++) sl[k] = (j - 2 * R + k) % NS;
       const int cy = D == 3 ? R + iy : 0;
       const int cx = R + ix;
-      T gx = 0, gy = 0, gz = 0;
-#pragma unroll
-      for (int e = 0; e < ES::QE; e++) {
-        const int em = D == 3 ? ES::ez[e] : ES::ey[e];
-        const int ey = D == 3 ? ES::ey[e] : 0;
-        const T v = lds[sl[R + em]][cy + ey][cx + ES::ex[e]];
-        const T w = T(ES::w[e]);
-        if (ES::ex[e] != 0) gx += T(ES::ex[e]) * w * v;
-        if (ES::ey[e] != 0) gy += T(ES::ey[e]) * w * v;
-        if (ES::ez[e] != 0) gz += T(ES::ez[e]) * w * v;
-      }
+      T gx, gy, gz;
+      iso_grad<ES>(
+          [&](int e) {
+            const int em = D == 3 ? ES::ez[e] : ES::ey[e];
+            const int ey = D == 3 ? ES::ey[e] : 0;
+            return lds[sl[R + em]][cy + ey][cx + ES::ex[e]];
+          },
+          gx, gy, gz);
       const T lpsi = lds[sl[R]][cy][cx];
       T fo[Q], u[3];
       collide<S, T, SHIFT, COLL>(fh[0], dnh[0], gx, gy, gz, lpsi, P, fo, u);
@@ -1244,17 +1287,14 @@ k_fused_dma(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<
         const int mc = m0 + j - 2 * R;
         const int cy = D == 3 ? R + iy : 0;
         const int cx = R + ix;
-        T gx = 0, gy = 0, gz = 0;
-#pragma unroll
-        for (int e = 0; e < ES::QE; e++) {
-          const int em = D == 3 ? ES::ez[e] : ES::ey[e];
-          const int ey = D == 3 ? ES::ey[e] : 0;
-          const T v = ring[(j - R + em) % NS][cy + ey][cx + ES::ex[e]];
-          const T w = T(ES::w[e]);
-          if (ES::ex[e] != 0) gx += T(ES::ex[e]) * w * v;
-          if (ES::ey[e] != 0) gy += T(ES::ey[e]) * w * v;
-          if (ES::ez[e] != 0) gz += T(ES::ez[e]) * w * v;
-        }
+        T gx, gy, gz;
+        iso_grad<ES>(
+            [&](int e) {
+              const int em = D == 3 ? ES::ez[e] : ES::ey[e];
+              const int ey = D == 3 ? ES::ey[e] : 0;
+              return ring[(j - R + em) % NS][cy + ey][cx + ES::ex[e]];
+            },
+            gx, gy, gz);
         const T lpsi = ring[(j - R) % NS][cy][cx];
         T u[3];
         collide<S, T, SHIFT, COLL, WALLS>(fh[0], dnh[0], gx, gy, gz, lpsi, PL, fpend, u, bx, by,
@@ -1330,18 +1370,14 @@ k_density_psi(const T* __restrict__ pop, Geom geo, Phys<T> P,
 template <class S, class ES, class T>
 __device__ inline void grad_global(const double* __restrict__ psi, const Geom& geo,
                                    int x, int y, int z, T& gx, T& gy, T& gz) {
-  gx = gy = gz = 0;
-#pragma unroll
-  for (int e = 0; e < ES::QE; e++) {
-    const int xn = ES::ex[e] ? wrap(x + ES::ex[e], geo.L0) : x;
-    const int yn = ES::ey[e] ? wrap(y + ES::ey[e], geo.L1) : y;
-    const int zn = ES::ez[e] ? wrap(z + ES::ez[e], geo.L2) : z;
-    const T v = (T)psi[lex(geo, xn, yn, zn)];
-    const T w = T(ES::w[e]);
-    if (ES::ex[e] != 0) gx += T(ES::ex[e]) * w * v;
-    if (ES::ey[e] != 0) gy += T(ES::ey[e]) * w * v;
-    if (ES::ez[e] != 0) gz += T(ES::ez[e]) * w * v;
-  }
+  iso_grad<ES>(
+      [&](int e) {
+        const int xn = ES::ex[e] ? wrap(x + ES::ex[e], geo.L0) : x;
+        const int yn = ES::ey[e] ? wrap(y + ES::ey[e], geo.L1) : y;
+        const int zn = ES::ez[e] ? wrap(z + ES::ez[e], geo.L2) : z;
+        return (T)psi[lex(geo, xn, yn, zn)];
+      },
+      gx, gy, gz);
 }
 
 __device__ inline void site_xyz(const Geom& geo, int64_t g, int& x, int& y, int& z) {
