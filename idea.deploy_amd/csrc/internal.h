@@ -32,6 +32,11 @@ struct idmx_ctx_s {
 
 struct SimOps;
 
+// Sites from which a 2D run on the x-shifted storage (variant 10, the default
+// launch there; the Shan-Chen forcing and the isotropy filter) takes two steps
+// per launch.
+constexpr int64_t kPairSites = 3 << 17;
+
 struct idmx_sc_s {
   idmx_ctx_s* ctx = nullptr;
   idmx_sc_desc desc{};

@@ -395,6 +395,7 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
   if (D == 2) {
     s->tx = d->dims[0] >= 256 ? 256 : 64;
     s->ty = 1;
+    if (V >= kPairSites) s->hist = 10;  // two steps per launch (Impl::pair_plan)
   } else {
     s->tx = 32;
     s->ty = 8;

@@ -3,8 +3,10 @@
 // which instantiate the combinations of their velocity set.
 #pragma once
 #include <algorithm>
+#include <cmath>
 
 #include "internal.h"
+#include "sc_pair.h"
 
 namespace idmx {
 
@@ -203,6 +205,77 @@ struct Impl {
   static constexpr bool kFixedDma3 =
       S::D == 3 && ES::R == 1 && DmaShape<S, ES, T, 64, 4, COLL>::fits;
 
+  // Two steps in one launch (k_pair2d): block width NT, columns written per
+  // block, rows marched.
+  struct PairPlan {
+    int nt = 0, txo = 0, H = 0;  // nt = 0: not on this lattice
+  };
+  // Two blocks of 256 (four of 128) share a CU; a launch takes about
+  // rounds * (H + 0.8 HALO) row times, the first and last HALO rows of a
+  // march being partly empty. Rows per block are even steps up to 40 (longer
+  // marches leave the last round unbalanced: 4096^2 E8 318 us per step at
+  // 32, 332 at 48), columns per block a multiple of 16 where that costs no
+  // further tile (2048^2: 75 us at 240 columns, 79 at 250). A half-filled
+  // chip runs a round in 0.68 of the time (1000 x 613: 14.9 us with 248
+  // blocks of 256, 15.5 with 927 of 128).
+  template <int NT>
+  static double pair_cost(const Geom& g, PairPlan& best, double least) {
+    using SH = PairShape<ES, T, COLL, NT>;
+    int ntx = (g.L0 + SH::TXMAX - 1) / SH::TXMAX;
+    const int even = ((g.L0 + ntx - 1) / ntx + 15) / 16 * 16;
+    const int txo = even <= SH::TXMAX ? even : SH::TXMAX;
+    ntx = (g.L0 + txo - 1) / txo;
+    for (int H = 4; H <= 40; H += 2) {
+      const double w = (double)ntx * ((g.L1 + H - 1) / H) / (512 * (256 / NT));
+      const double rounds = w <= 0.5 ? 0.68 : w <= 3 ? std::ceil(w) : w + 0.5;
+      const double c = rounds * (H + 0.8 * SH::HALO);
+      if (c < least) {
+        least = c;
+        best = {NT, txo, H};
+      }
+    }
+    return least;
+  }
+  // Below 3 * 2^17 sites the march is a chain of too few blocks: 512^2 10.8 us
+  // per step against 10.8 with single steps, 256^2 9.5 against 6.4 (1024^2
+  // MRT: 21.8 against 38.6). A lattice much narrower than a block leaves its
+  // lanes idle.
+  static PairPlan pair_plan(const idmx_sc_s* s) {
+    PairPlan p;
+    if constexpr (S::D == 2)
+      if (s->geo.V >= kPairSites) {
+        const double c = pair_cost<256>(s->geo, p, 1e300);
+        pair_cost<128>(s->geo, p, c);
+        const int ntx = (s->geo.L0 + p.txo - 1) / p.txo;
+        if (2 * s->geo.L0 < ntx * p.nt) p.nt = 0;
+      }
+    return p;
+  }
+  template <int NT, bool WF>
+  static hipError_t launch_pair(idmx_sc_s* s, const PairPlan& p, const T* pop, T* swap, double* n,
+                                double* psi, double* u) {
+    if constexpr (S::D == 2) {
+      const Geom& g = s->geo;
+      const int ntx = (g.L0 + p.txo - 1) / p.txo, H = std::min(p.H, g.L1);
+      const int ntiles = ntx * ((g.L1 + H - 1) / H);
+      const unsigned grid = (unsigned)((ntiles + 7) / 8 * 8);
+      hipLaunchKernelGGL((k_pair2d<ES, T, SHIFT, COLL, NT, WF>), dim3(grid), dim3(NT), 0,
+                         s->ctx->stream, pop, swap, g, phys(s), p.txo, H, ntx, ntiles, s->xsh, n,
+                         psi, u);
+      return hipGetLastError();
+    } else {
+      return hipErrorInvalidConfiguration;
+    }
+  }
+  static hipError_t pair(idmx_sc_s* s, const PairPlan& p, const T* pop, T* swap, double* n,
+                         double* psi, double* u) {
+    if (p.nt == 128)
+      return n ? launch_pair<128, true>(s, p, pop, swap, n, psi, u)
+               : launch_pair<128, false>(s, p, pop, swap, n, psi, u);
+    return n ? launch_pair<256, true>(s, p, pop, swap, n, psi, u)
+             : launch_pair<256, false>(s, p, pop, swap, n, psi, u);
+  }
+
   // Tile shapes the autotuner chooses from; the step that writes n/psi/u at
   // a checkpoint uses one fixed shape.
   template <bool WF>
@@ -326,7 +399,27 @@ struct Impl {
       IDMX_HIP(hipGetLastError());
       std::swap(*pop, *swap);
     }
-    for (int k = 0; k < nsteps; k++) {
+    // two steps per launch: an even number of pairs, so that the state ends in
+    // the buffer in which single steps would leave it
+    const PairPlan pp = S::D == 2 && xs && !twop && !fwalls && !pev ? pair_plan(s) : PairPlan{};
+    const int npair = pp.nt ? nsteps / 2 & ~1 : 0;
+    if (npair > 0) {
+      const int nl = nsteps - npair;  // single steps first, then the pairs
+      for (int k = 0; k < nl; k++) {
+        const T* a = (const T*)*pop;
+        T* b = (T*)*swap;
+        s->xsh = (k > 0 ? 1 : 0) | (k < nl - 1 ? 2 : 0);
+        const bool f = wf && k == nl - 1;
+        hipError_t e;
+        if (k >= nl - npair) e = pair(s, pp, a, b, f ? n : nullptr, psi, u);
+        else if constexpr (COLL >= 3) e = fused_fixed<false>(s, a, b, nullptr, nullptr, nullptr);
+        else e = fused<false>(s, a, b, nullptr, nullptr, nullptr);
+        s->xsh = 0;
+        if (e != hipSuccess) return hip_fail(e, "idmx_sc_run launch");
+        std::swap(*pop, *swap);
+      }
+    }
+    for (int k = npair > 0 ? nsteps : 0; k < nsteps; k++) {
       const bool last = k == nsteps - 1;
       const T* a = (const T*)*pop;
       T* b = (T*)*swap;

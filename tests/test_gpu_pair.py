@@ -1,0 +1,68 @@
+"""Two steps per launch (k_pair2d, 2D lattices of at least 3 * 2^17 sites on
+variant 10 and with the Shan-Chen forcing or the isotropy filter) against
+single steps: variant 9, or the two-pass step for the forcing and the filter.
+Every site sees the same arithmetic, so FP64 results are equal and FP32 ones
+may differ by the contraction of a few operations per step. Sizes lie at the
+edges of the tiles (250 / 246 and 122 / 118 columns written per block), with
+rows that leave a remainder; runs of 4 to 7 steps have 2 pairs and 0 to 3
+single steps, and 3 steps none."""
+import numpy as np
+import pytest
+
+from helpers import droplet_field
+
+pytestmark = pytest.mark.gpu
+
+CASES = [('D2E4', (500, 787), 'fp64', 'bgk'), ('D2E4', (251, 1571), 'fp64', 'mrt'),
+         ('D2E8', (493, 801), 'fp64', 'bgk'), ('D2E6', (4099, 97), 'fp64', 'dense'),
+         ('D2E4', (123, 3201), 'fp64', 'bgk'), ('D2E4', (1499, 263), 'fp64', 'sc'),
+         ('D2E8', (613, 643), 'fp64', 'iso'), ('D2E4', (749, 526), 'fp32s', 'bgk'),
+         ('D2E8', (640, 615), 'fp32s', 'mrt')]
+
+
+def _run(tenet, es, dims, prec, coll, single, steps, wf):
+    from idmx.IdpyCode import IdpyMemory
+    from idmx.LBM import hermite
+    from idmx.LBM._base import PopArray
+    from idmx.LBM._engine import SCEngine
+    S = np.diag(np.linspace(0.7, 1.5, 9))
+    if coll == 'dense':
+        S[3, 4] = 0.05
+    kw = {'mrt': hermite.mrt_kernel_tables('D2Q9', S)} if coll in ('mrt', 'dense') else \
+        {'forcing': 'sc'} if coll == 'sc' else {'iso_filter': True} if coll == 'iso' else {}
+    eng = SCEngine(tenet, 'D2Q9', es, dims, 'exp', -5.0 / 3.0, 1.0, precision=prec, rho0=1.0,
+                   **kw)
+    assert eng.get_launch()[3] == 10
+    if single:
+        eng.set_launch(64, 1, 8, 9)
+    V = eng.V
+    n = IdpyMemory.OnDevice(droplet_field(dims, seed=21), tenet)
+    psi = IdpyMemory.Zeros(V, np.float64, tenet)
+    u = IdpyMemory.Zeros(2 * V, np.float64, tenet)
+    a, b = PopArray(eng, tenet), PopArray(eng, tenet)
+    eng.init_pop(a, n, u)
+    swapped = eng.run(a, b, steps, n=n, psi=psi, u=u, write_fields=wf,
+                      two_pass=single and coll in ('sc', 'iso'))
+    out = [(b if swapped else a).RawD2H()]
+    if wf:
+        out += [n.D2H(), psi.D2H(), u.D2H()]
+    for x in (a, b, n, psi, u):
+        x.Free()
+    eng.close()
+    return swapped, out
+
+
+@pytest.mark.parametrize('es,dims,prec,coll', CASES)
+@pytest.mark.parametrize('steps,wf', [(3, True), (4, True), (5, False), (6, True), (7, True),
+                                      (8, False)])
+def test_two_steps_per_launch_equal_single_steps(tenet, es, dims, prec, coll, steps, wf):
+    sw1, ref = _run(tenet, es, dims, prec, coll, True, steps, wf)
+    sw2, got = _run(tenet, es, dims, prec, coll, False, steps, wf)
+    assert sw1 == sw2      # the state ends in the buffer where single steps leave it
+    for r, g in zip(ref, got):
+        assert np.isfinite(g).all()
+        if prec == 'fp64':
+            assert np.array_equal(r, g)
+        else:
+            # ~10 roundings of 6e-8 of the largest value per step
+            assert np.abs(r - g).max() <= steps * 10 * 6e-8 * np.abs(r).max()
