@@ -29,13 +29,17 @@ FLAGS = ['-std=c++17', '-O3', '-fPIC', '--offload-arch=' + ARCH,
 # without floating-point contraction, as the reference's CTypes backend
 # computes: with fused multiply-adds the FP64 trajectory drifts from it by
 # 2e-11 over 10^4 steps, without by 1e-13. The FP32-shifted lattice units
-# (single-domain and batched) and the network kernels keep contraction.
+# (single-domain and batched) contract within an expression only: across
+# expressions (hipcc's default, which the network kernels keep) the choice of
+# fused operations differs from kernel to kernel, and with it the last bits of
+# the same step in another launch shape.
 NOFMA = ['-ffp-contract=off']
-SOURCES = [('runtime.hip', NOFMA), ('sc_d2q9.hip', NOFMA), ('sc_d2q9_f32.hip', []),
-           ('sc_d3q19_e4.hip', NOFMA), ('sc_d3q19_e4_f32.hip', []),
-           ('sc_d3q19_e6.hip', NOFMA), ('sc_d3q19_e6_f32.hip', []),
-           ('sc_d3q19_e8.hip', NOFMA), ('sc_d3q19_e8_f32.hip', []),
-           ('batch.hip', NOFMA), ('batch_f32.hip', []), ('nn.hip', []), ('noalloc.hip', NOFMA),
+INEXPR = ['-ffp-contract=on']
+SOURCES = [('runtime.hip', NOFMA), ('sc_d2q9.hip', NOFMA), ('sc_d2q9_f32.hip', INEXPR),
+           ('sc_d3q19_e4.hip', NOFMA), ('sc_d3q19_e4_f32.hip', INEXPR),
+           ('sc_d3q19_e6.hip', NOFMA), ('sc_d3q19_e6_f32.hip', INEXPR),
+           ('sc_d3q19_e8.hip', NOFMA), ('sc_d3q19_e8_f32.hip', INEXPR),
+           ('batch.hip', NOFMA), ('batch_f32.hip', INEXPR), ('nn.hip', []), ('noalloc.hip', NOFMA),
            ('init_fields.hip', NOFMA)]
 
 
