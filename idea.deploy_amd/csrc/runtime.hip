@@ -409,6 +409,41 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
     const int blocks_at_8 = ntx * nty * ((Lm + 7) / 8);
     H = std::max(H, blocks_at_8 >= 256 ? 8 : (D == 2 ? 1 : 2));
     s->H = std::min(H, Lm);
+    // 3D lattices that fill the chip: the LDS-staged step on the x-shifted
+    // storage. Two of its blocks share a CU, so the launch runs in rounds of
+    // 512 blocks of H + 2R planes each, and the tile and H with the least
+    // total win (one full round where the lattice allows it: 150 x 101 x 93
+    // 127 us per step at 32 x 8, H = 14, 455 blocks, against 142 at H = 8;
+    // 200^3 MRT 592 us at 64 x 4, H = 40, against 816 with registers). A
+    // plane of 32 x 8 takes 6 % longer than one of 64 x 4 (shorter rows), but
+    // pads less on most widths. Reach-2 stencils in FP64 leave one block per
+    // CU and stay on registers (96^3 E8: 86 us against 131), as does the dense
+    // MRT collision, which is bound by its 741 products (128^3: 503 us against
+    // 556) and lattices of a few planes per block (48 x 44 x 40: 14.2 us
+    // against 17.4; 64^3 FP32: 14.1 against 15.4).
+    const bool f32 = d->precision == IDMX_PREC_F32S;
+    if (D == 3 && (R == 1 || f32) && s->coll != 1 && V >= (f32 ? 500000 : 200000)) {
+      double least = 1e300;
+      for (int tx : {64, 32}) {
+        const int ty = 256 / tx;
+        // the Shan-Chen forcing runs 64 x 4 tiles (Impl::fused_fixed)
+        if ((tx == 32 && s->coll == 3) || !s->ops->launch_ok(tx, ty, 10)) continue;
+        const int64_t tiles =
+            (int64_t)((s->geo.L0 + tx - 1) / tx) * ((s->geo.L1 + ty - 1) / ty);
+        for (int nseg = 1; nseg <= std::min(Lm, 4096); nseg++) {
+          const int h = (Lm + nseg - 1) / nseg;
+          const int64_t rounds = (tiles * ((Lm + h - 1) / h) + 511) / 512;
+          const double c = (double)rounds * (h + 2 * R + 0.5) * (tx == 32 ? 1.06 : 1.0);
+          if (c < least) {
+            least = c;
+            s->tx = tx;
+            s->ty = ty;
+            s->H = h;
+            s->hist = 10;
+          }
+        }
+      }
+    }
   }
   if (d->collision == IDMX_MRT) {
     const int NB = D == 2 ? 6 : 10;
