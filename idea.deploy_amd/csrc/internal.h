@@ -28,6 +28,8 @@ struct idmx_ctx_s {
   double* partials = nullptr;      // device scratch for reductions
   size_t partials_cap = 0;         // in doubles
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  float* nn_part = nullptr;        // per-block weight gradients of the network
+  size_t nn_part_cap = 0;          // in floats; grown on demand, freed with the context
 };
 
 struct SimOps;

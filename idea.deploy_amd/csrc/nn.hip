@@ -17,26 +17,9 @@
 #include <algorithm>
 
 #include "internal.h"
+#include "nn_conv.h"
 
 namespace idmx {
-
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef float v4f32 __attribute__((ext_vector_type(4)));
-
-__device__ inline float bf2f(uint16_t b) {
-  return __uint_as_float(((uint32_t)b) << 16);
-}
-// round to nearest even
-__device__ inline uint16_t f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7f800000u) == 0x7f800000u) return (uint16_t)(u >> 16);  // inf / nan
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
-
-struct ConvShape {
-  int N, H, W, Cin, Cout;
-};
 
 // ---------------------------------------------------------------------------
 // Forward 3x3 convolution, stride 1, zero padding 1:
@@ -378,6 +361,106 @@ inline unsigned g1(int64_t n, int bs = 256) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + bs - 1) / bs, 65536));
 }
 
+inline bool aligned(const void* p, size_t n) { return ((uintptr_t)p & (n - 1)) == 0; }
+
+template <int CIN, int TP>
+hipError_t conv_tile_ct(idmx_ctx_s* c, const void* in, const void* wt, const float* bias,
+                        void* out, float* out_f32, const ConvShape& s, int relu, int ct) {
+  const int P = s.N * s.H * s.W, cots = (s.Cout + 15) / 16;
+  const dim3 grid((P + TP - 1) / TP, cots / ct);
+  const size_t shm = ConvTile<CIN>::lds(s.W, TP);
+  auto go = [&](auto k) {
+    hipLaunchKernelGGL(k, grid, dim3(256), shm, c->stream, (const uint16_t*)in,
+                       (const uint16_t*)wt, bias, (uint16_t*)out, out_f32, s, relu);
+    return hipGetLastError();
+  };
+  if (ct == 4) return go(k_conv3x3_tile<CIN, 4, TP>);
+  if (ct == 2) return go(k_conv3x3_tile<CIN, 2, TP>);
+  return go(k_conv3x3_tile<CIN, 1, TP>);
+}
+
+// The tiled convolution where it applies (its channel counts, 16-byte rows,
+// staged rows within 64 KB): 256 pixels per block where that makes 256 blocks
+// or more, else 64; as many output-channel tiles per block as leave 512
+// blocks. Other shapes run k_conv3x3_fwd.
+template <int CIN>
+bool conv_tile(idmx_ctx_s* c, const void* in, const void* wt, const float* bias, void* out,
+               float* out_f32, const ConvShape& s, int relu, hipError_t& e) {
+  const int P = s.N * s.H * s.W, cots = (s.Cout + 15) / 16;
+  int ct = cots % 4 == 0 ? 4 : cots % 2 == 0 ? 2 : 1;
+  const bool big = ConvTile<CIN>::lds(s.W, 256) <= 65536 &&
+                   (int64_t)(P + 255) / 256 * (cots / ct) >= 256;
+  const int tp = big ? 256 : 64;
+  if (ConvTile<CIN>::lds(s.W, tp) > 65536) return false;
+  while (ct > 1 && (int64_t)(P + tp - 1) / tp * (cots / ct) < 512) ct /= 2;
+  e = big ? conv_tile_ct<CIN, 256>(c, in, wt, bias, out, out_f32, s, relu, ct)
+          : conv_tile_ct<CIN, 64>(c, in, wt, bias, out, out_f32, s, relu, ct);
+  return true;
+}
+
+hipError_t conv_fwd(idmx_ctx_s* c, const void* in, const void* wt, const float* bias, void* out,
+                    float* out_f32, const ConvShape& s, int relu) {
+  hipError_t e = hipSuccess;
+  if (aligned(in, 16) && aligned(wt, 8)) {
+    bool done = false;
+    switch (s.Cin) {
+      case 8: done = conv_tile<8>(c, in, wt, bias, out, out_f32, s, relu, e); break;
+      case 16: done = conv_tile<16>(c, in, wt, bias, out, out_f32, s, relu, e); break;
+      case 32: done = conv_tile<32>(c, in, wt, bias, out, out_f32, s, relu, e); break;
+      case 64: done = conv_tile<64>(c, in, wt, bias, out, out_f32, s, relu, e); break;
+      case 128: done = conv_tile<128>(c, in, wt, bias, out, out_f32, s, relu, e); break;
+    }
+    if (done) return e;
+  }
+  const int64_t waves = (int64_t)((s.N * s.H * s.W + 15) / 16) * ((s.Cout + 15) / 16);
+  hipLaunchKernelGGL(k_conv3x3_fwd, dim3(g1(waves * 64)), dim3(256), 0, c->stream,
+                     (const uint16_t*)in, (const uint16_t*)wt, bias, (uint16_t*)out, out_f32, s,
+                     relu);
+  return hipGetLastError();
+}
+
+// The tiled backward-weight where it applies; false: not this shape.
+template <int CIN, int COUT>
+bool bwd_w_tile(idmx_ctx_s* c, const void* in, const void* dy, float* dw, float* db,
+                const ConvShape& s, hipError_t& e) {
+  using B = BwdW<CIN, COUT>;
+  if (s.W % 4 || B::TPX % s.W || B::lds(s.W) > 160 * 1024) return false;
+  const int P = s.N * s.H * s.W, nchunks = (P + B::TPX - 1) / B::TPX;
+  const int blocks = std::min(nchunks, 512), nw = COUT * 9 * CIN;
+  const size_t need = (size_t)blocks * (nw + COUT);
+  if (need > c->nn_part_cap) {
+    if (c->nn_part) {
+      e = hipStreamSynchronize(c->stream);
+      if (e == hipSuccess) e = hipFree(c->nn_part);
+      if (e != hipSuccess) return true;
+    }
+    c->nn_part = nullptr;
+    c->nn_part_cap = 0;
+    e = hipMalloc(&c->nn_part, need * sizeof(float));
+    if (e != hipSuccess) return true;
+    c->nn_part_cap = need;
+  }
+  hipLaunchKernelGGL((k_conv3x3_bwd_w_tile<CIN, COUT>), dim3(blocks), dim3(256), B::lds(s.W),
+                     c->stream, (const uint16_t*)in, (const uint16_t*)dy, c->nn_part, s, nchunks);
+  hipLaunchKernelGGL(k_conv_bwd_w_sum, dim3((nw + COUT + 63) / 64), dim3(256), 0, c->stream,
+                     c->nn_part, dw, db, nw, COUT, blocks);
+  e = hipGetLastError();
+  return true;
+}
+
+template <int CIN>
+bool bwd_w_cout(idmx_ctx_s* c, const void* in, const void* dy, float* dw, float* db,
+                const ConvShape& s, hipError_t& e) {
+  switch (s.Cout) {
+    case 1: return bwd_w_tile<CIN, 1>(c, in, dy, dw, db, s, e);
+    case 16: return bwd_w_tile<CIN, 16>(c, in, dy, dw, db, s, e);
+    case 32: return bwd_w_tile<CIN, 32>(c, in, dy, dw, db, s, e);
+    case 64:
+      if constexpr (CIN <= 64) return bwd_w_tile<CIN, 64>(c, in, dy, dw, db, s, e);
+  }
+  return false;
+}
+
 }  // namespace idmx
 
 using namespace idmx;
@@ -397,12 +480,7 @@ int idmx_nn_conv3x3_fwd(idmx_ctx_t c, const void* in, const void* wt, const floa
                         int relu) {
   NCHECK(c && in && wt && out && N > 0 && H > 0 && W > 0 && Cin > 0 && Cout > 0,
          "idmx_nn_conv3x3_fwd: invalid argument");
-  ConvShape s{N, H, W, Cin, Cout};
-  const int64_t waves = (int64_t)((N * H * W + 15) / 16) * ((Cout + 15) / 16);
-  hipLaunchKernelGGL(k_conv3x3_fwd, dim3(g1(waves * 64)), dim3(256), 0, c->stream,
-                     (const uint16_t*)in, (const uint16_t*)wt, bias, (uint16_t*)out, out_f32, s,
-                     relu);
-  IDMX_HIP(hipGetLastError());
+  IDMX_HIP(conv_fwd(c, in, wt, bias, out, out_f32, ConvShape{N, H, W, Cin, Cout}, relu));
   return IDMX_OK;
 }
 
@@ -413,12 +491,7 @@ int idmx_nn_conv3x3_bwd_data(idmx_ctx_t c, const void* dy, const float* w, void*
   const int tot = Cin * 9 * Cout;
   hipLaunchKernelGGL(k_conv_flip_weights, dim3(g1(tot)), dim3(256), 0, c->stream, w,
                      (uint16_t*)wd_scratch, Cin, Cout);
-  ConvShape s{N, H, W, Cout, Cin};
-  const int64_t waves = (int64_t)((N * H * W + 15) / 16) * ((Cin + 15) / 16);
-  hipLaunchKernelGGL(k_conv3x3_fwd, dim3(g1(waves * 64)), dim3(256), 0, c->stream,
-                     (const uint16_t*)dy, (const uint16_t*)wd_scratch, (const float*)nullptr,
-                     (uint16_t*)dx, (float*)nullptr, s, 0);
-  IDMX_HIP(hipGetLastError());
+  IDMX_HIP(conv_fwd(c, dy, wd_scratch, nullptr, dx, nullptr, ConvShape{N, H, W, Cout, Cin}, 0));
   return IDMX_OK;
 }
 
@@ -426,6 +499,21 @@ int idmx_nn_conv3x3_bwd_weight(idmx_ctx_t c, const void* in, const void* dy, flo
                                float* db, int N, int H, int W, int Cin, int Cout) {
   NCHECK(c && in && dy && dw, "idmx_nn_conv3x3_bwd_weight: invalid argument");
   ConvShape s{N, H, W, Cin, Cout};
+  if (aligned(in, 16) && aligned(dy, 16)) {
+    hipError_t e = hipSuccess;
+    bool done = false;
+    switch (Cin) {
+      case 8: done = bwd_w_cout<8>(c, in, dy, dw, db, s, e); break;
+      case 16: done = bwd_w_cout<16>(c, in, dy, dw, db, s, e); break;
+      case 32: done = bwd_w_cout<32>(c, in, dy, dw, db, s, e); break;
+      case 64: done = bwd_w_cout<64>(c, in, dy, dw, db, s, e); break;
+      case 128: done = bwd_w_cout<128>(c, in, dy, dw, db, s, e); break;
+    }
+    if (done) {
+      IDMX_HIP(e);
+      return IDMX_OK;
+    }
+  }
   const int P = N * H * W;
   const int pchunk = 1024;
   const int64_t waves = (int64_t)((Cout + 15) / 16) * ((9 * Cin + 15) / 16) *

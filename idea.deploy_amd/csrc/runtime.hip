@@ -184,6 +184,7 @@ int idmx_ctx_destroy(idmx_ctx_t c) {
   hipSetDevice(c->device);
   if (c->stream) hipStreamSynchronize(c->stream);
   if (c->partials) hipFree(c->partials);
+  if (c->nn_part) hipFree(c->nn_part);
   if (c->ev0) hipEventDestroy(c->ev0);
   if (c->ev1) hipEventDestroy(c->ev1);
   if (c->stream) hipStreamDestroy(c->stream);
