@@ -30,13 +30,20 @@ struct ConvShape {
 // Forward 3x3 convolution of TP consecutive pixels (in (n, y, x) order) by CT
 // tiles of 16 output channels per block; the arithmetic of k_conv3x3_fwd, in
 // its order (16 k values per MFMA, k = tap * CIN + ci ascending), so the two
-// agree bit for bit.
+// agree bit for bit. The weights are the MFMA's rows and the pixels its
+// columns, so a lane ends with 4 output channels of one pixel (8-byte stores).
+//
+// Bound by latency at these sizes (a layer of the batch-32 network is 0.3 to
+// 1.2 GFLOP and 1 to 25 MB): a wave's weights, at most 144 registers, are
+// requested before the rows are staged, so one latency covers both, and the
+// loop over taps reads LDS only.
 template <int CIN>
 struct ConvTile {
   // dwords between pixels in LDS: 16 lanes read 16 consecutive pixels, 8
   // dwords each, and these strides spread them over all 64 banks
   static constexpr int SD = CIN == 8 ? 4 : CIN == 16 ? 8 : CIN == 32 ? 24 : CIN / 2 + 4;
   static constexpr int ZERO = 3 * SD;  // dwords of a zero area
+  static constexpr int CTMAX = CIN <= 16 ? 4 : CIN == 32 ? 2 : 1;
   static int rows(int W, int tp) { return (tp + W - 2) / W + 1 + 2; }
   static size_t lds(int W, int tp) {
     return 4 * ((size_t)rows(W, tp) * (W + 2) * SD + ZERO);
@@ -50,6 +57,7 @@ k_conv3x3_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict__ wt,
                float* __restrict__ out_f32, ConvShape s, int relu) {
   using C = ConvTile<CIN>;
   constexpr int SD = C::SD, K = 9 * CIN, NM = TP / 64;  // 16-pixel tiles per wave
+  constexpr int NSL = (K + 15) / 16;                    // MFMAs along k
   extern __shared__ uint32_t lds[];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int P = s.N * s.H * s.W, W = s.W;
@@ -57,32 +65,69 @@ k_conv3x3_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict__ wt,
   const int row0 = p0 / W - 1;  // first staged row, rows counted over all images
   const int nrows = (min(p0 + TP, P) - 1) / W + 1 - row0 + 1;
   const int nr_all = s.N * s.H;
-  uint32_t* stage = lds + C::ZERO;
+  const int r = lane & 15, kq = lane >> 4;
+  const int ct0 = blockIdx.y * CT;
 
-  // stage the rows, with a zero pixel at both ends, 8 channels per access
-  constexpr int CH = CIN / 8;
-  const int cols = W + 2, total = nrows * cols * CH;
+  v4i16 wf[NSL][CT];
+#pragma unroll
+  for (int c = 0; c < CT; c++) {
+    const int co = (ct0 + c) * 16 + r;
+    const uint16_t* w = wt + (int64_t)(co < s.Cout ? co : 0) * K + 4 * kq;
+#pragma unroll
+    for (int i = 0; i < NSL; i++) {
+      wf[i][c] = v4i16{0, 0, 0, 0};
+      if (co < s.Cout && (K % 16 == 0 || 16 * i + 4 * kq < K)) wf[i][c] = *(const v4i16*)(w + 16 * i);
+    }
+  }
+
+  // stage the rows, with a zero pixel at both ends, 8 channels per access and
+  // U accesses per thread in flight (one at a time: 21 us instead of 16 for
+  // 16 -> 16 channels of 128 64 x 64 images)
+  constexpr int CH = CIN / 8, U = CIN <= 16 ? 4 : 8;
+  const int cols = W + 2, rowlen = cols * CH;
   for (int i = tid; i < C::ZERO; i += 256) lds[i] = 0;
-  for (int i = tid; i < total; i += 256) {
-    const int c8 = i % CH, t = i / CH;
-    const int col = t % cols, row = t / cols;
-    const int g = row0 + row, x = col - 1;
-    v4u32 v = {0, 0, 0, 0};
-    if (g >= 0 && g < nr_all && x >= 0 && x < W)
-      v = *(const v4u32*)(in + ((int64_t)g * W + x) * CIN + c8 * 8);
-    *(v4u32*)(stage + (row * cols + col) * SD + c8 * 4) = v;
+  for (int row = 0, i = tid; row < nrows;) {
+    v4u32 v[U];
+    int dst[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      while (i >= rowlen) {
+        i -= rowlen;
+        row++;
+      }
+      const int x = i / CH - 1, c8 = i % CH, g = row0 + row;
+      v[u] = v4u32{0, 0, 0, 0};
+      dst[u] = row < nrows ? C::ZERO + (row * cols + x + 1) * SD + c8 * 4 : -1;
+      if (row < nrows && g >= 0 && g < nr_all && x >= 0 && x < W)
+        v[u] = *(const v4u32*)(in + ((int64_t)g * W + x) * CIN + c8 * 8);
+      i += 256;
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (dst[u] >= 0) *(v4u32*)(lds + dst[u]) = v[u];
+    while (i >= rowlen && row < nrows) {
+      i -= rowlen;
+      row++;
+    }
   }
   __syncthreads();
 
-  const int r = lane & 15, kq = lane >> 4;
-  const int ct0 = blockIdx.y * CT;
   // LDS dword of the pixel left of this lane's pixel in the rows above, at and
   // below it; rows outside its image read the zero area
   uint32_t ra[NM][3];
+  int p = p0 + wv * NM * 16 + r;
+  int g = p / W, x = p - g * W, y = g % s.H;  // stepped by 16 pixels below
 #pragma unroll
   for (int m = 0; m < NM; m++) {
-    const int p = p0 + (wv * NM + m) * 16 + r;
-    const int g = p / W, x = p - g * W, y = g % s.H;
+    if (m > 0) {
+      p += 16;
+      x += 16;
+      while (x >= W) {
+        x -= W;
+        g++;
+        y = y + 1 == s.H ? 0 : y + 1;
+      }
+    }
 #pragma unroll
     for (int d = 0; d < 3; d++) {
       const bool ok = p < P && y + d - 1 >= 0 && y + d - 1 < s.H;
@@ -90,80 +135,60 @@ k_conv3x3_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict__ wt,
       if (CIN >= 16) ra[m][d] += 2 * kq;
     }
   }
-  const uint16_t* wb[CT];
-  bool cv[CT];
-#pragma unroll
-  for (int c = 0; c < CT; c++) {
-    const int co = (ct0 + c) * 16 + r;
-    cv[c] = co < s.Cout;
-    wb[c] = wt + (int64_t)(cv[c] ? co : 0) * K + 4 * kq;
-  }
   v4f32 acc[NM][CT];
 #pragma unroll
   for (int m = 0; m < NM; m++)
 #pragma unroll
     for (int c = 0; c < CT; c++) acc[m][c] = {0.f, 0.f, 0.f, 0.f};
-  auto ldw = [&](int c, int k) {
-    v4i16 b = {0, 0, 0, 0};
-    if (cv[c] && (K % 16 == 0 || k + 4 * kq < K)) b = *(const v4i16*)(wb[c] + k);
-    return b;
-  };
-  if constexpr (CIN >= 16) {
 #pragma unroll
-    for (int dy = 0; dy < 3; dy++)
+  for (int i = 0; i < NSL; i++)
 #pragma unroll
-      for (int dx = 0; dx < 3; dx++)
-#pragma unroll
-        for (int c0 = 0; c0 < CIN; c0 += 16) {
-          v4i16 b[CT];
-#pragma unroll
-          for (int c = 0; c < CT; c++) b[c] = ldw(c, (3 * dy + dx) * CIN + c0);
-#pragma unroll
-          for (int m = 0; m < NM; m++) {
-            const v4i16 a = *(const v4i16*)(lds + ra[m][dy] + dx * SD + c0 / 2);
-#pragma unroll
-            for (int c = 0; c < CT; c++)
-              acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[c], acc[m][c], 0, 0, 0);
-          }
-        }
-  } else {
-    // 8 channels: an MFMA's 16 k values are two taps
-#pragma unroll
-    for (int t0 = 0; t0 < 10; t0 += 2) {
-      v4i16 b[CT];
-#pragma unroll
-      for (int c = 0; c < CT; c++) b[c] = ldw(c, t0 * 8);
-      const int tap = t0 + (kq >> 1);
-      const int dy = tap >= 9 ? 0 : tap / 3, dx = tap >= 9 ? 0 : tap % 3;
-#pragma unroll
-      for (int m = 0; m < NM; m++) {
+    for (int m = 0; m < NM; m++) {
+      v4i16 a;
+      if constexpr (CIN >= 16) {
+        const int tap = 16 * i / CIN, c0 = 16 * i % CIN;
+        a = *(const v4i16*)(lds + ra[m][tap / 3] + tap % 3 * SD + c0 / 2);
+      } else {
+        // 8 channels: an MFMA's 16 k values are two taps
+        const int tap = 2 * i + (kq >> 1);
+        const int dy = tap >= 9 ? 0 : tap / 3, dx = tap >= 9 ? 0 : tap % 3;
         const uint32_t base = dy == 0 ? ra[m][0] : dy == 1 ? ra[m][1] : ra[m][2];
-        v4i16 a = *(const v4i16*)(lds + base + dx * SD + 2 * (kq & 1));
+        a = *(const v4i16*)(lds + base + dx * SD + 2 * (kq & 1));
         if (tap >= 9) a = v4i16{0, 0, 0, 0};
+      }
 #pragma unroll
-        for (int c = 0; c < CT; c++)
-          acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[c], acc[m][c], 0, 0, 0);
+      for (int c = 0; c < CT; c++)
+        acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wf[i][c], a, acc[m][c], 0, 0, 0);
+    }
+  // D: column = lane % 16 (pixel), rows 4 * (lane / 16) + j (output channels)
+#pragma unroll
+  for (int m = 0; m < NM; m++) {
+    const int64_t p = p0 + (wv * NM + m) * 16 + r;
+    if (p >= P) continue;
+#pragma unroll
+    for (int c = 0; c < CT; c++) {
+      const int oc = (ct0 + c) * 16 + 4 * kq;
+      v4f32 v = acc[m][c];
+      if ((s.Cout & 3) == 0) {
+        if (oc >= s.Cout) continue;
+        if (bias) v += *(const v4f32*)(bias + oc);
+        if (out_f32) *(v4f32*)(out_f32 + p * s.Cout + oc) = v;
+        uint16_t h[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) h[j] = f2bf(relu ? fmaxf(v[j], 0.f) : v[j]);
+        *(v2u32*)(out + p * s.Cout + oc) =
+            v2u32{h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16};
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          if (oc + j < s.Cout) {
+            float t = v[j] + (bias ? bias[oc + j] : 0.f);
+            if (out_f32) out_f32[p * s.Cout + oc + j] = t;
+            if (relu) t = fmaxf(t, 0.f);
+            out[p * s.Cout + oc + j] = f2bf(t);
+          }
       }
     }
-  }
-  // D: column = lane % 16 (output channel), rows 4 * (lane / 16) + j (pixels)
-#pragma unroll
-  for (int c = 0; c < CT; c++) {
-    const int oc = (ct0 + c) * 16 + r;
-    if (oc >= s.Cout) continue;
-    const float bv = bias ? bias[oc] : 0.f;
-#pragma unroll
-    for (int m = 0; m < NM; m++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int op = p0 + (wv * NM + m) * 16 + 4 * kq + j;
-        if (op < P) {
-          float v = acc[m][c][j] + bv;
-          if (out_f32) out_f32[(int64_t)op * s.Cout + oc] = v;
-          if (relu) v = fmaxf(v, 0.f);
-          out[(int64_t)op * s.Cout + oc] = f2bf(v);
-        }
-      }
   }
 }
 
@@ -178,9 +203,8 @@ k_conv3x3_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict__ wt,
 // each side, dY as [co][pixel]. One read of the 8 pixels x - 2 .. x + 5 serves
 // the three taps of a row (the taps at x - 1 and x + 1 are 16-bit shifts of
 // it).
-template <int CIN, int COUT>
+template <int CIN, int COUT, int TPX>
 struct BwdW {
-  static constexpr int TPX = 256;
   static constexpr int CI = (CIN + 15) / 16, CO = (COUT + 15) / 16;  // 16 x 16 tiles
   // waves: over input-channel tiles first, then output-channel tiles, then
   // groups of pixels (summed over LDS at the end)
@@ -200,15 +224,29 @@ struct BwdW {
   }
 };
 
+// 8 bf16 values of g where those of y are positive, else 0
+__device__ __forceinline__ v4u32 relu_mask(v4u32 y, v4u32 g) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint32_t lo = __uint_as_float(y[i] << 16) > 0.f ? 0xffffu : 0u;
+    const uint32_t hi = __uint_as_float(y[i] & 0xffff0000u) > 0.f ? 0xffff0000u : 0u;
+    g[i] &= lo | hi;
+  }
+  return g;
+}
+
 // 16-bit pairs (hi of a, lo of b) -> dword
 __device__ __forceinline__ uint32_t mid16(uint32_t a, uint32_t b) { return (a >> 16) | (b << 16); }
 
-template <int CIN, int COUT>
+// With y (the layer's ReLU output) dY is masked by y > 0 first, in place: a
+// block stages every channel of its pixels, each exactly once.
+template <int CIN, int COUT, int TPX>
 __global__ void __launch_bounds__(256)
-k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict__ dy,
-                     float* __restrict__ part, ConvShape s, int nchunks) {
-  using B = BwdW<CIN, COUT>;
-  constexpr int TPX = B::TPX, NI = B::NI, NO = B::NO, YP = B::YP;
+k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, uint16_t* __restrict__ dy,
+                     const uint16_t* __restrict__ y, float* __restrict__ part, ConvShape s,
+                     int nchunks) {
+  using B = BwdW<CIN, COUT, TPX>;
+  constexpr int NI = B::NI, NO = B::NO, YP = B::YP;
   extern __shared__ uint32_t lds[];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int W = s.W, H = s.H, P = s.N * H * W;
@@ -218,6 +256,7 @@ k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict
   const int r = lane & 15, kq = lane >> 4;
   const int wi = wv % B::WI, wo = wv / B::WI % B::WO, wp = wv / (B::WI * B::WO);
   const int nr_all = s.N * H;
+  const int lq4 = 31 - __builtin_clz(W / 4);
   if (tid < 4) lds[tid] = 0;
   // the zero pixels at both ends of every staged row
   for (int i = tid; i < CIN * nrows; i += 256) {
@@ -238,11 +277,11 @@ k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict
     const int p0 = ch * TPX, row0 = p0 / W - 1;
     __syncthreads();
     // X: 4 pixels x 8 channels per thread and round, transposed in registers
+    // (row and column by shifts: W / 4 is a power of two, as W divides TPX)
     constexpr int CH = CIN / 8;
-    const int q4 = W / 4;
-    for (int i = tid; i < nrows * q4 * CH; i += 256) {
+    for (int i = tid; i < (nrows << lq4) * CH; i += 256) {
       const int c8 = i % CH, t = i / CH;
-      const int x4 = t % q4, row = t / q4, g = row0 + row;
+      const int x4 = t & ((1 << lq4) - 1), row = t >> lq4, g = row0 + row;
       v4u32 v[4];
 #pragma unroll
       for (int k = 0; k < 4; k++) {
@@ -268,8 +307,14 @@ k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict
 #pragma unroll
         for (int k = 0; k < 4; k++) {
           v[k] = v4u32{0, 0, 0, 0};
-          if (p0 + 4 * p4 + k < P)
-            v[k] = *(const v4u32*)(dy + (int64_t)(p0 + 4 * p4 + k) * COUT + c8 * 8);
+          if (p0 + 4 * p4 + k < P) {
+            const int64_t o = (int64_t)(p0 + 4 * p4 + k) * COUT + c8 * 8;
+            v[k] = *(const v4u32*)(dy + o);
+            if (y) {
+              v[k] = relu_mask(*(const v4u32*)(y + o), v[k]);
+              *(v4u32*)(dy + o) = v[k];
+            }
+          }
         }
 #pragma unroll
         for (int c = 0; c < 8; c++) {
@@ -282,7 +327,13 @@ k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict
     } else {
       for (int i = tid; i < TPX * COUT; i += 256) {
         const int c = i % COUT, p = i / COUT;
-        ((uint16_t*)(ys + c * YP))[p] = p0 + p < P ? dy[(int64_t)(p0 + p) * COUT + c] : 0;
+        const int64_t o = (int64_t)(p0 + p) * COUT + c;
+        uint16_t v = p0 + p < P ? dy[o] : (uint16_t)0;
+        if (y && p0 + p < P) {
+          v = bf2f(y[o]) > 0.f ? v : (uint16_t)0;
+          dy[o] = v;
+        }
+        ((uint16_t*)(ys + c * YP))[p] = v;
       }
     }
     __syncthreads();
@@ -298,7 +349,7 @@ k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict
     }
     for (int px = wp * 16; px < TPX; px += 16 * B::WP) {
       const int pq = px + 4 * kq, p = p0 + pq;  // this lane's 4 pixels
-      const int g = p / W, x = p - g * W, y = g % H;
+      const int g = p / W, x = p - g * W, yr = g % H;
       v4i16 a[NO];
 #pragma unroll
       for (int o = 0; o < NO; o++) {
@@ -311,7 +362,7 @@ k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict
         const uint32_t cb = 4 + (CIN % 16 == 0 || ci < CIN ? ci : ci - CIN) * plane + x / 2;
 #pragma unroll
         for (int d = 0; d < 3; d++) {
-          const bool ok = p < P && y + d - 1 >= 0 && y + d - 1 < H;
+          const bool ok = p < P && yr + d - 1 >= 0 && yr + d - 1 < H;
           const uint32_t* src = lds + (ok ? cb + (g + d - 1 - row0) * rw : 0u);
           const uint32_t w0 = src[0], w1 = src[1], w2 = src[2], w3 = src[3];
           const uint32_t m01 = mid16(w0, w1), m12 = mid16(w1, w2), m23 = mid16(w2, w3);
@@ -375,21 +426,41 @@ k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict
         }
 }
 
-// dw[i] += sum_b part[b][i] (i < nw), db[i - nw] likewise (db may be null)
+// dw[i] += sum_b part[b][i] (i < nw), db[i - nw] likewise (db may be null): 64
+// sums per block, its four waves over a quarter of the parts each, eight loads
+// in flight. The blocks past those (fl of them) write the weights for the
+// backward-data pass instead, the transposed, tap-flipped kernel
+// wd[ci][tap' Cout + co] = w[co][(8 - tap') Cin + ci] in bf16.
 __global__ void __launch_bounds__(256)
 k_conv_bwd_w_sum(const float* __restrict__ part, float* __restrict__ dw, float* __restrict__ db,
-                 int nw, int nb, int blocks) {
+                 int nw, int nb, int blocks, const float* __restrict__ w,
+                 uint16_t* __restrict__ wd, int Cin, int Cout) {
+  const int n = nw + nb, sums = (n + 63) / 64;
+  if ((int)blockIdx.x >= sums) {
+    const int i = (blockIdx.x - sums) * 256 + threadIdx.x;
+    if (i < nw) {
+      const int ci = i / (9 * Cout), rem = i % (9 * Cout);
+      const int tp = rem / Cout, co = rem % Cout;
+      wd[i] = f2bf(w[(int64_t)co * 9 * Cin + (8 - tp) * Cin + ci]);
+    }
+    return;
+  }
   const int i = blockIdx.x * 64 + (threadIdx.x & 63), g = threadIdx.x >> 6;
   __shared__ float f[4][64];
-  float v = 0.f;
-  if (i < nw + nb)
-    for (int b = g; b < blocks; b += 4) v += part[(int64_t)b * (nw + nb) + i];
-  f[g][threadIdx.x & 63] = v;
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (i < n) {
+    int b = g;
+    for (; b + 28 < blocks; b += 32)
+#pragma unroll
+      for (int k = 0; k < 8; k++) v[k] += part[(int64_t)(b + 4 * k) * n + i];
+    for (; b < blocks; b += 4) v[0] += part[(int64_t)b * n + i];
+  }
+  f[g][threadIdx.x & 63] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   __syncthreads();
-  if (g == 0 && i < nw + nb) {
-    v = f[0][threadIdx.x] + f[1][threadIdx.x] + f[2][threadIdx.x] + f[3][threadIdx.x];
-    if (i < nw) dw[i] += v;
-    else if (db) db[i - nw] += v;
+  if (g == 0 && i < n) {
+    const float t = (f[0][threadIdx.x] + f[1][threadIdx.x]) + (f[2][threadIdx.x] + f[3][threadIdx.x]);
+    if (i < nw) dw[i] += t;
+    else if (db) db[i - nw] += t;
   }
 }
 

@@ -118,13 +118,18 @@ _SIGS = [
     ('idmx_nn_conv3x3_fwd', C.c_int, [C.c_void_p] * 6 + [C.c_int] * 6),
     ('idmx_nn_conv3x3_bwd_data', C.c_int, [C.c_void_p] * 5 + [C.c_int] * 5),
     ('idmx_nn_conv3x3_bwd_weight', C.c_int, [C.c_void_p] * 5 + [C.c_int] * 5),
+    ('idmx_nn_conv3x3_bwd', C.c_int, [C.c_void_p] * 9 + [C.c_int] * 5),
     ('idmx_nn_relu_bwd', C.c_int, [C.c_void_p] * 4 + [C.c_int64]),
     ('idmx_nn_pool2', C.c_int, [C.c_void_p] * 3 + [C.c_int] * 5),
     ('idmx_nn_up2', C.c_int, [C.c_void_p] * 3 + [C.c_int] * 7),
     ('idmx_nn_copy_channels', C.c_int, [C.c_void_p] * 3 + [C.c_int64] + [C.c_int] * 5),
+    ('idmx_nn_cat_up2', C.c_int, [C.c_void_p] * 4 + [C.c_int] * 5),
+    ('idmx_nn_pool2_bwd_add', C.c_int, [C.c_void_p] * 5 + [C.c_int] * 6),
     ('idmx_nn_add', C.c_int, [C.c_void_p] * 4 + [C.c_int64]),
     ('idmx_nn_mse', C.c_int, [C.c_void_p] * 4 + [C.c_int64, c_double_p]),
     ('idmx_nn_adam', C.c_int, [C.c_void_p] * 6 + [C.c_int64] + [C.c_float] * 4 + [C.c_int]),
+    ('idmx_nn_adam_set', C.c_int, [C.c_void_p, C.c_int] + [c_void_pp] * 5
+     + [C.POINTER(C.c_int64)] + [C.c_float] * 4 + [C.c_int]),
     ('idmx_nn_cast', C.c_int, [C.c_void_p] * 3 + [C.c_int64, C.c_int]),
     ('idmx_nn_resize_to_lattice', C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p,
                                             C.c_int, C.c_double]),

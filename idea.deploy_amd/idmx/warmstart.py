@@ -194,15 +194,10 @@ class UNet:
         """dout_key holds dL/d(output); applies the ReLU mask in place, adds
         dL/dW, dL/db, and writes dL/d(input) into din_key."""
         L = self.layers[name]
-        n = self.N * s * s * L['co']
-        if L['relu']:
-            _lib.call('idmx_nn_relu_bwd', self.h, self.a[name].ptr, self.a[dout_key].ptr,
-                      self.a[dout_key].ptr, n)
-        _lib.call('idmx_nn_conv3x3_bwd_weight', self.h, self.a[src].ptr, self.a[dout_key].ptr,
-                  L['g'].ptr, L['gb'].ptr, self.N, s, s, L['ci'], L['co'])
-        if need_din:
-            _lib.call('idmx_nn_conv3x3_bwd_data', self.h, self.a[dout_key].ptr, L['w'].ptr,
-                      L['wd'].ptr, self.a[din_key].ptr, self.N, s, s, L['ci'], L['co'])
+        _lib.call('idmx_nn_conv3x3_bwd', self.h, self.a[src].ptr,
+                  self.a[name].ptr if L['relu'] else None, self.a[dout_key].ptr, L['w'].ptr,
+                  L['wd'].ptr, self.a[din_key].ptr if need_din else None, L['g'].ptr, L['gb'].ptr,
+                  self.N, s, s, L['ci'], L['co'])
 
     def _pool(self, src, dst, s, c, bwd=0):
         _lib.call('idmx_nn_pool2', self.h, self.a[src].ptr, self.a[dst].ptr, self.N, s, s, c, bwd)
@@ -211,19 +206,22 @@ class UNet:
         _lib.call('idmx_nn_up2', self.h, self.a[src].ptr, self.a[dst].ptr, self.N, s, s, c, cy,
                   c0, bwd)
 
-    def _copy(self, src, dst, P, cx, cx0, cy, cy0, c):
-        _lib.call('idmx_nn_copy_channels', self.h, self.a[src].ptr, self.a[dst].ptr, P, cx, cx0,
-                  cy, cy0, c)
+    def _cat(self, src, skip, dst, s, c, cs):
+        """dst = [2x upsample of src (s x s, c channels), skip (cs channels)]"""
+        _lib.call('idmx_nn_cat_up2', self.h, self.a[src].ptr, self.a[skip].ptr, self.a[dst].ptr,
+                  self.N, s, s, c, cs)
 
-    def _add(self, a, b, y, n):
-        _lib.call('idmx_nn_add', self.h, self.a[a].ptr, self.a[b].ptr, self.a[y].ptr, n)
+    def _pool_skip_bwd(self, dpool, dcat, dst, s, c, cc, c0):
+        """Gradient of a tensor that feeds a pool and a skip connection."""
+        _lib.call('idmx_nn_pool2_bwd_add', self.h, self.a[dpool].ptr, self.a[dcat].ptr,
+                  self.a[dst].ptr, self.a['tmp'].ptr, self.N, s, s, c, cc, c0)
 
     # -- forward / backward -------------------------------------------------
     def set_input(self, x_bf16):
         self.a['x'].h2d(x_bf16)
 
     def forward(self):
-        N, s = self.N, S
+        s = S
         self._conv('c1a', 'x', 'c1a', s)
         self._conv('c1b', 'c1a', 'c1b', s)
         self._pool('c1b', 'p1', s, 16)
@@ -235,16 +233,13 @@ class UNet:
         self._pool('c3b', 'p3', s // 4, 64)
         self._conv('c4a', 'p3', 'c4a', s // 8)
         self._conv('c4b', 'c4a', 'c4b', s // 8)
-        self._up('c4b', 'cat3', s // 8, 64, 128, 0)
-        self._copy('c3b', 'cat3', N * (s // 4) ** 2, 64, 0, 128, 64, 64)
+        self._cat('c4b', 'c3b', 'cat3', s // 8, 64, 64)
         self._conv('d3a', 'cat3', 'd3a', s // 4)
         self._conv('d3b', 'd3a', 'd3b', s // 4)
-        self._up('d3b', 'cat2', s // 4, 32, 64, 0)
-        self._copy('c2b', 'cat2', N * (s // 2) ** 2, 32, 0, 64, 32, 32)
+        self._cat('d3b', 'c2b', 'cat2', s // 4, 32, 32)
         self._conv('d2a', 'cat2', 'd2a', s // 2)
         self._conv('d2b', 'd2a', 'd2b', s // 2)
-        self._up('d2b', 'cat1', s // 2, 16, 32, 0)
-        self._copy('c1b', 'cat1', N * s * s, 16, 0, 32, 16, 16)
+        self._cat('d2b', 'c1b', 'cat1', s // 2, 16, 16)
         self._conv('d1a', 'cat1', 'd1a', s)
         self._conv('d1b', 'd1a', 'd1b', s)
         self._conv('head', 'd1b', 'head', s, out32=self.out32)
@@ -256,7 +251,7 @@ class UNet:
         return loss.value
 
     def backward(self):
-        N, s = self.N, S
+        s = S
         self._conv_bwd('head', 'd1b', 'dhead', 'dd1b', s)
         self._conv_bwd('d1b', 'd1a', 'dd1b', 'dd1a', s)
         self._conv_bwd('d1a', 'cat1', 'dd1a', 'dcat1', s)
@@ -270,33 +265,26 @@ class UNet:
         self._conv_bwd('c4b', 'c4a', 'dc4b', 'dc4a', s // 8)
         self._conv_bwd('c4a', 'p3', 'dc4a', 'dp3', s // 8)
         # c3b feeds the pool and the skip into cat3
-        self._pool('dp3', 'dc3b', s // 4, 64, bwd=1)
-        P3 = N * (s // 4) ** 2
-        self._copy('dcat3', 'tmp', P3, 128, 64, 64, 0, 64)
-        self._add('dc3b', 'tmp', 'dc3b', P3 * 64)
+        self._pool_skip_bwd('dp3', 'dcat3', 'dc3b', s // 4, 64, 128, 64)
         self._conv_bwd('c3b', 'c3a', 'dc3b', 'dc3a', s // 4)
         self._conv_bwd('c3a', 'p2', 'dc3a', 'dp2', s // 4)
-        self._pool('dp2', 'dc2b', s // 2, 32, bwd=1)
-        P2 = N * (s // 2) ** 2
-        self._copy('dcat2', 'tmp', P2, 64, 32, 32, 0, 32)
-        self._add('dc2b', 'tmp', 'dc2b', P2 * 32)
+        self._pool_skip_bwd('dp2', 'dcat2', 'dc2b', s // 2, 32, 64, 32)
         self._conv_bwd('c2b', 'c2a', 'dc2b', 'dc2a', s // 2)
         self._conv_bwd('c2a', 'p1', 'dc2a', 'dp1', s // 2)
-        self._pool('dp1', 'dc1b', s, 16, bwd=1)
-        P1 = N * s * s
-        self._copy('dcat1', 'tmp', P1, 32, 16, 16, 0, 16)
-        self._add('dc1b', 'tmp', 'dc1b', P1 * 16)
+        self._pool_skip_bwd('dp1', 'dcat1', 'dc1b', s, 16, 32, 16)
         self._conv_bwd('c1b', 'c1a', 'dc1b', 'dc1a', s)
         self._conv_bwd('c1a', 'x', 'dc1a', 'dx', s, need_din=False)
 
     def adam(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):
         self.step += 1
-        for L in self.layers.values():
-            nw = L['co'] * 9 * L['ci']
-            _lib.call('idmx_nn_adam', self.h, L['w'].ptr, L['g'].ptr, L['m'].ptr, L['v'].ptr,
-                      L['wb'].ptr, nw, lr, b1, b2, eps, self.step)
-            _lib.call('idmx_nn_adam', self.h, L['b'].ptr, L['gb'].ptr, L['mb'].ptr, L['vb'].ptr,
-                      None, L['co'], lr, b1, b2, eps, self.step)
+        ls = list(self.layers.values())
+        arr = lambda t, v: (t * len(v))(*v)
+        ptrs = [arr(C.c_void_p, [L[k].ptr.value for L in ls] + [L[kb].ptr.value for L in ls])
+                for k, kb in (('w', 'b'), ('g', 'gb'), ('m', 'mb'), ('v', 'vb'))]
+        wb = arr(C.c_void_p, [L['wb'].ptr.value for L in ls] + [None] * len(ls))
+        n = arr(C.c_int64, [L['co'] * 9 * L['ci'] for L in ls] + [L['co'] for L in ls])
+        _lib.call('idmx_nn_adam_set', self.h, 2 * len(ls), *ptrs, wb, n, lr, b1, b2, eps,
+                  self.step)
 
     # -- host helpers -------------------------------------------------------
     def get_weights(self):

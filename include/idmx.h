@@ -457,6 +457,13 @@ int idmx_nn_conv3x3_bwd_data(idmx_ctx_t ctx, const void* dy, const float* w,
 int idmx_nn_conv3x3_bwd_weight(idmx_ctx_t ctx, const void* in, const void* dy,
                                float* dw, float* db, int N, int H, int W,
                                int Cin, int Cout);
+/* One layer's backward pass: with y (the layer's ReLU output, or NULL) dy is
+ * masked in place first, then dw and db as idmx_nn_conv3x3_bwd_weight and dx
+ * (NULL: not wanted) as idmx_nn_conv3x3_bwd_data; fewer launches than the
+ * three calls. */
+int idmx_nn_conv3x3_bwd(idmx_ctx_t ctx, const void* in, const void* y, void* dy,
+                        const float* w, void* wd_scratch, void* dx, float* dw,
+                        float* db, int N, int H, int W, int Cin, int Cout);
 int idmx_nn_relu_bwd(idmx_ctx_t ctx, const void* y, const void* dy, void* dx,
                      int64_t n);
 /* 2x2 average pool (bwd = 0: x is N,H,W,C -> y N,H/2,W/2,C; bwd = 1: x is the
@@ -471,6 +478,16 @@ int idmx_nn_up2(idmx_ctx_t ctx, const void* x, void* y, int N, int H, int W,
                 int C, int Cy, int c0, int bwd);
 int idmx_nn_copy_channels(idmx_ctx_t ctx, const void* x, void* y, int64_t P,
                           int Cx, int cx0, int Cy, int cy0, int C);
+/* y (N,2H,2W,C+Cs) = nearest 2x upsample of x (N,H,W,C), then skip
+ * (N,2H,2W,Cs), along the channels. */
+int idmx_nn_cat_up2(idmx_ctx_t ctx, const void* x, const void* skip, void* y,
+                    int N, int H, int W, int C, int Cs);
+/* dx (N,H,W,C) = the 2x2 average pool's gradient of dpool (N,H/2,W/2,C) plus
+ * channels [c0, c0+C) of dcat (N,H,W,Cc), the first rounded to bf16 before
+ * the sum; scratch holds N*H*W*C bf16 values. */
+int idmx_nn_pool2_bwd_add(idmx_ctx_t ctx, const void* dpool, const void* dcat,
+                          void* dx, void* scratch, int N, int H, int W, int C,
+                          int Cc, int c0);
 int idmx_nn_add(idmx_ctx_t ctx, const void* a, const void* b, void* y,
                 int64_t n);
 /* loss = mean (pred - tgt)^2, grad = 2 (pred - tgt) / n in bf16. */
@@ -481,6 +498,12 @@ int idmx_nn_mse(idmx_ctx_t ctx, const float* pred, const float* tgt,
 int idmx_nn_adam(idmx_ctx_t ctx, float* w, float* g, float* m, float* v,
                  void* wb, int64_t n, float lr, float b1, float b2, float eps,
                  int t);
+/* idmx_nn_adam for `count` tensors (host arrays of device pointers and
+ * lengths; wb[k] may be NULL) in one launch per 32. */
+int idmx_nn_adam_set(idmx_ctx_t ctx, int count, float* const* w, float* const* g,
+                     float* const* m, float* const* v, void* const* wb,
+                     const int64_t* n, float lr, float b1, float b2, float eps,
+                     int t);
 /* float32 <-> bf16 */
 int idmx_nn_cast(idmx_ctx_t ctx, const void* x, void* y, int64_t n,
                  int to_bf16);
