@@ -38,6 +38,8 @@ struct SimOps;
 // launch there; the Shan-Chen forcing and the isotropy filter) takes two steps
 // per launch.
 constexpr int64_t kPairSites = 3 << 17;
+// Steps per launch below that (E4 force).
+constexpr int kTileSteps = 4;
 
 struct idmx_sc_s {
   idmx_ctx_s* ctx = nullptr;

@@ -396,7 +396,9 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
   if (D == 2) {
     s->tx = d->dims[0] >= 256 ? 256 : 64;
     s->ty = 1;
-    if (V >= kPairSites) s->hist = 10;  // two steps per launch (Impl::pair_plan)
+    // several steps per launch: two on large lattices (Impl::pair_plan), four
+    // on small ones with the E4 force (Impl::tile)
+    if (V >= kPairSites || R == 1) s->hist = 10;
   } else {
     s->tx = 32;
     s->ty = 8;

@@ -7,6 +7,7 @@
 
 #include "internal.h"
 #include "sc_pair.h"
+#include "sc_tile.h"
 
 namespace idmx {
 
@@ -276,6 +277,44 @@ struct Impl {
              : launch_pair<256, false>(s, p, pop, swap, n, psi, u);
   }
 
+  // One 2D step with the populations held in registers.
+  static hipError_t fused_regs(idmx_sc_s* s, const T* pop, T* swap) {
+    if constexpr (S::D == 2) {
+      if (s->geo.L0 >= 256)
+        return launch_fused<256, 1, false, true>(s, pop, swap, nullptr, nullptr, nullptr);
+      return launch_fused<64, 1, false, true>(s, pop, swap, nullptr, nullptr, nullptr);
+    } else {
+      return hipErrorInvalidConfiguration;
+    }
+  }
+
+  // Four steps in one launch on a small 2D lattice (k_tile2d).
+  static constexpr bool kTile = S::D == 2 && ES::R == 1;
+  template <int B, bool WF>
+  static hipError_t launch_tile(idmx_sc_s* s, const T* pop, T* swap, double* n, double* psi,
+                                double* u) {
+    const Geom& g = s->geo;
+    const int ntx = (g.L0 + B - 1) / B, ntiles = ntx * ((g.L1 + B - 1) / B);
+    const unsigned grid = (unsigned)((ntiles + 7) / 8 * 8);
+    hipLaunchKernelGGL((k_tile2d<T, SHIFT, COLL, B, kTileSteps, WF>), dim3(grid),
+                       dim3(TileShape<B, kTileSteps>::NT), 0, s->ctx->stream, pop, swap, g,
+                       phys(s), ntx, ntiles, n, psi, u);
+    return hipGetLastError();
+  }
+  static hipError_t tile(idmx_sc_s* s, const T* pop, T* swap, double* n, double* psi, double* u) {
+    if constexpr (kTile) {
+      // 8 x 8 tiles while every one has a CU of its own (128^2: 1.92 us per
+      // step against 2.50), else 16 x 16 (256^2: 2.53 against 4.24)
+      if ((int64_t)((s->geo.L0 + 7) / 8) * ((s->geo.L1 + 7) / 8) <= 256)
+        return n ? launch_tile<8, true>(s, pop, swap, n, psi, u)
+                 : launch_tile<8, false>(s, pop, swap, n, psi, u);
+      return n ? launch_tile<16, true>(s, pop, swap, n, psi, u)
+               : launch_tile<16, false>(s, pop, swap, n, psi, u);
+    } else {
+      return hipErrorInvalidConfiguration;
+    }
+  }
+
   // Tile shapes the autotuner chooses from; the step that writes n/psi/u at
   // a checkpoint uses one fixed shape.
   template <bool WF>
@@ -391,7 +430,10 @@ struct Impl {
     // steps reads the streamed storage, the last writes it (the step that
     // writes n/psi/u runs on the streamed storage), so a run of one step
     // never leaves it
-    const bool xs = fwalls || (COLL < 3 ? s->hist == 10 : (kFixedDma2 || kFixedDma3));
+    // (small 2D lattices with the E4 force stay on the streamed storage on
+    // variant 10: kTileSteps steps per launch, single steps with registers)
+    const bool small = kTile && !fwalls && s->geo.V < kPairSites;
+    const bool xs = fwalls || (COLL < 3 ? s->hist == 10 && !small : (kFixedDma2 || kFixedDma3));
     const int nxsh = xs && !twop ? nsteps - (wf ? 1 : 0) : 0;
     if constexpr (COLL < 3) if (pull) {
       hipLaunchKernelGGL((k_restream<S, T>), dim3(grid_for(s->geo.V)), dim3(256), 0, st,
@@ -419,7 +461,28 @@ struct Impl {
         std::swap(*pop, *swap);
       }
     }
-    for (int k = npair > 0 ? nsteps : 0; k < nsteps; k++) {
+    // kTileSteps steps per launch, an even number of such launches for the same
+    // reason; they and the single steps before them keep the streamed storage
+    int nquad = 0;
+    if constexpr (kTile)
+      if (small && !twop && !pev && (COLL >= 3 || s->hist == 10))
+        nquad = nsteps / kTileSteps & ~1;
+    if constexpr (kTile)
+      if (nquad > 0) {
+        const int nl = nsteps - nquad * (kTileSteps - 1);
+        for (int k = 0; k < nl; k++) {
+          const T* a = (const T*)*pop;
+          T* b = (T*)*swap;
+          const bool f = wf && k == nl - 1;
+          const hipError_t e =
+              k >= nl - nquad
+                  ? tile(s, a, b, f ? n : nullptr, psi, u)
+                  : fused_regs(s, a, b);
+          if (e != hipSuccess) return hip_fail(e, "idmx_sc_run launch");
+          std::swap(*pop, *swap);
+        }
+      }
+    for (int k = npair > 0 || nquad > 0 ? nsteps : 0; k < nsteps; k++) {
       const bool last = k == nsteps - 1;
       const T* a = (const T*)*pop;
       T* b = (T*)*swap;
@@ -451,6 +514,7 @@ struct Impl {
           if (mid) IDMX_HIP(hipEventRecord(mid, st));
           s->xsh = k < nxsh ? (k > 0 ? 1 : 0) | (k < nxsh - 1 ? 2 : 0) : 0;
           if (wf && last) e = fused<true>(s, a, b, n, psi, u);
+          else if (small && s->hist == 10) e = fused_regs(s, a, b);
           else e = fused<false>(s, a, b, nullptr, nullptr, nullptr);
           s->xsh = 0;
         }

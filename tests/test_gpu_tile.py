@@ -1,0 +1,67 @@
+"""Four steps per launch on small 2D lattices (k_tile2d: E4 force, fewer than
+3 * 2^17 sites, the default launch) against single steps with the populations
+in registers (variant 1), or against the two-pass step for the Shan-Chen
+forcing and the isotropy filter: the same arithmetic per site, equal in FP64
+and, contraction being the same in every launch, to rounding in FP32. Lattices
+smaller than a tile and its ring, edges of the 8 x 8 and 16 x 16 tiles, and
+runs that leave single steps over."""
+import numpy as np
+import pytest
+
+from helpers import droplet_field
+
+pytestmark = pytest.mark.gpu
+
+CASES = [((3, 3), 'fp64', 'bgk'), ((5, 70), 'fp64', 'mrt'), ((128, 128), 'fp64', 'bgk'),
+         ((127, 129), 'fp64', 'bgk'), ((129, 145), 'fp64', 'dense'), ((17, 300), 'fp64', 'sc'),
+         ((8, 16), 'fp64', 'iso'), ((301, 47), 'fp64', 'bgk'), ((627, 627), 'fp64', 'mrt'),
+         ((95, 64), 'fp32s', 'bgk'), ((161, 200), 'fp32s', 'mrt')]
+
+
+def _run(tenet, dims, prec, coll, single, steps, wf):
+    from idmx.IdpyCode import IdpyMemory
+    from idmx.LBM import hermite
+    from idmx.LBM._base import PopArray
+    from idmx.LBM._engine import SCEngine
+    S = np.diag(np.linspace(0.7, 1.5, 9))
+    if coll == 'dense':
+        S[3, 4] = 0.05
+    kw = {'mrt': hermite.mrt_kernel_tables('D2Q9', S)} if coll in ('mrt', 'dense') else \
+        {'forcing': 'sc'} if coll == 'sc' else {'iso_filter': True} if coll == 'iso' else {}
+    eng = SCEngine(tenet, 'D2Q9', 'D2E4', dims, 'exp', -5.0 / 3.0, 1.0, precision=prec,
+                   rho0=1.0, **kw)
+    assert eng.get_launch()[3] == 10
+    if single:
+        eng.set_launch(64, 1, 3, 1)
+    V = eng.V
+    n0 = droplet_field(dims, seed=4) if min(dims) > 20 else \
+        1.0 + 0.3 * np.sin(2 * np.pi * np.arange(V) / max(dims) + 0.3)
+    n = IdpyMemory.OnDevice(n0, tenet)
+    psi = IdpyMemory.Zeros(V, np.float64, tenet)
+    u = IdpyMemory.Zeros(2 * V, np.float64, tenet)
+    a, b = PopArray(eng, tenet), PopArray(eng, tenet)
+    eng.init_pop(a, n, u)
+    swapped = eng.run(a, b, steps, n=n, psi=psi, u=u, write_fields=wf,
+                      two_pass=single and coll in ('sc', 'iso'))
+    out = [(b if swapped else a).RawD2H()]
+    if wf:
+        out += [n.D2H(), psi.D2H()] + ([u.D2H()] if prec == 'fp64' else [])
+    for x in (a, b, n, psi, u):
+        x.Free()
+    eng.close()
+    return swapped, out
+
+
+@pytest.mark.parametrize('dims,prec,coll', CASES)
+@pytest.mark.parametrize('steps,wf', [(7, True), (8, True), (8, False), (13, True), (18, False)])
+def test_four_steps_per_launch_equal_single_steps(tenet, dims, prec, coll, steps, wf):
+    sw1, ref = _run(tenet, dims, prec, coll, True, steps, wf)
+    sw2, got = _run(tenet, dims, prec, coll, False, steps, wf)
+    assert sw1 == sw2      # the state ends in the buffer where single steps leave it
+    for r, g in zip(ref, got):
+        assert np.isfinite(g).all()
+        if prec == 'fp64':
+            assert np.array_equal(r, g)
+        else:
+            # ~10 roundings of 6e-8 of the largest value per step
+            assert np.abs(r - g).max() <= steps * 10 * 6e-8 * np.abs(r).max()
