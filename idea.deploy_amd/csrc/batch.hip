@@ -186,6 +186,17 @@ int idmx_batch_create(idmx_ctx_t ctx, const idmx_batch_domain* doms, int ndom, i
   hipDeviceProp_t p;
   hipGetDeviceProperties(&p, ctx->device);
   b->grid = p.multiProcessorCount * 8;
+  // With the E4 force two steps per launch on the x-shifted storage (64
+  // domains of 64^2 to 256^2, FP64: 42.8 us per step with 16 x 16 tiles, 73.2
+  // with the one-step 32 x 8 ones; one domain of 128^2: 3.3 against 4.1).
+  // FP32 keeps three blocks of 32 x 16 per CU, which re-read less, as long as
+  // there are enough of them (22.0 against 24.2 us at 32 x 8).
+  if (estencil == IDMX_E4) {
+    b->kind = 5;
+    const bool wide = precision == IDMX_PREC_F32S && so >= 200000;
+    b->tx = wide ? 32 : 16;
+    b->H = 16;
+  }
   int rc = rebuild_items(b);
   if (rc) {
     idmx_batch_destroy(b);
@@ -226,7 +237,10 @@ int idmx_batch_set_launch(idmx_batch_t b, int kind, int tx, int H, int grid) {
   b->kind = kind;
   b->tx = tx;
   b->H = H;
-  if (grid > 0) b->grid = grid;
+  if (grid > 0) {
+    b->grid = grid;
+    b->grid_auto = false;
+  }
   drop_graph(b);
   return rebuild_items(b);
 }

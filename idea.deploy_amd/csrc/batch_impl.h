@@ -35,6 +35,11 @@ struct idmx_batch_s {
   unsigned long long* d_dmax = nullptr;
   int max_items = 0, n_items = 0;
   int grid = 0;
+  // no idmx_batch_set_launch yet with a grid: a step launch has one block per
+  // live item, which the dispatcher balances better than blocks striding over
+  // the items (64 domains of 64^2 to 256^2, kind 5: 42.8 us per step against
+  // 48.5 with 2048 blocks; E8, kind 1: 69.8 against 76.2)
+  bool grid_auto = true;
   hipGraphExec_t graph = nullptr;
   int graph_steps = 0;
   int graph_grid = 0;  // step grid the graph was captured with
@@ -48,7 +53,7 @@ namespace idmx {
 // work item. The step kernels order their items per XCD (xcd_block), which
 // spreads the items over all XCDs only when no block is surplus.
 inline int step_grid(const idmx_batch_s* b) {
-  return std::max(1, std::min(b->grid, b->n_items));
+  return std::max(1, b->grid_auto ? b->n_items : std::min(b->grid, b->n_items));
 }
 
 template <class ES, class T, bool SHIFT, int TX, bool PULL>
