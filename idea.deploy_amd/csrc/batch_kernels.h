@@ -68,11 +68,13 @@ __device__ inline void march2d(const T* __restrict__ pop, T* __restrict__ pop_sw
       lds[slot][R + tid] = psi_of(P.psi_kind, SHIFT ? P.rho0 + s : s);
     }
     if (has_halo) {
-      T s = 0;
+      T fhalo[Q];
 #pragma unroll
       for (int q = 0; q < Q; q++)
-        s += pop[(size_t)q * geo.V +
-                 (PULL ? pull_src<S>(geo, q, (int)halo_off, 0, mj) : base + halo_off)];
+        fhalo[q] = pop[(size_t)q * geo.V +
+                       (PULL ? pull_src<S>(geo, q, (int)halo_off, 0, mj) : base + halo_off)];
+      arrive(fhalo);
+      const T s = pop_sum(fhalo);
       lds[slot][hx] = psi_of(P.psi_kind, SHIFT ? P.rho0 + s : s);
     }
     __syncthreads();
@@ -203,10 +205,12 @@ k_batched_tile(const T* __restrict__ pop_all, T* __restrict__ swap_all,
       }
       const int hxs = pmod(w.x0 - R + hx, d.L0), hys = pmod(w.m0 - R + hy, d.L1);
       const int64_t g = (int64_t)hys * d.L0 + hxs;
-      T sh = 0;
+      T fh[Q];
 #pragma unroll
       for (int q = 0; q < Q; q++)
-        sh += pop[(size_t)q * geo.V + (PULL ? pull_src<S>(geo, q, hxs, 0, hys) : g)];
+        fh[q] = pop[(size_t)q * geo.V + (PULL ? pull_src<S>(geo, q, hxs, 0, hys) : g)];
+      arrive(fh);
+      const T sh = pop_sum(fh);
       lds[hy][hx] = psi_of(P.psi_kind, SHIFT ? P.rho0 + sh : sh);
     }
     __syncthreads();

@@ -41,6 +41,13 @@ constexpr int64_t kPairSites = 3 << 17;
 // Steps per launch below that (E4 force).
 constexpr int kTileSteps = 4;
 
+// Sites below which a 3D simulation that was given no launch takes its steps
+// without a march (k_tile3d): 24^3 MRT 7.6 us per step against 13.1, 48 x 44 x
+// 40 11.6 against 14.1 (E8: 16.5 against 19.5), 60 x 50 x 48 BGK 19.3 against
+// 21.4, 64^3 25.9 against 23.6; in FP32 48 x 44 x 40 8.4 against 10.4, 50^3
+// 13.7 against 12.7.
+constexpr int64_t kTile3Sites = 150000, kTile3Sites32 = 100000;
+
 struct idmx_sc_s {
   idmx_ctx_s* ctx = nullptr;
   idmx_sc_desc desc{};
@@ -54,6 +61,7 @@ struct idmx_sc_s {
   const SimOps* ops = nullptr;
   // fused launch shape (chosen at create time, autotuner may override)
   int tx = 0, ty = 0, H = 0, hist = 1;
+  bool auto_launch = true;  // no idmx_sc_set_launch yet
   int xsh = 0;  // variant 10: the running step's x-shifted storage flags
   int coll = 0;  // 0 BGK, 1 dense MRT, 2 diagonal MRT, 3 BGK with Shan-Chen forcing,
                  // 4 BGK followed by the isotropy filter

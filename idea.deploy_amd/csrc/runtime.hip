@@ -518,6 +518,7 @@ int idmx_sc_set_launch(idmx_sc_t s, int tx, int ty, int H, int hist) {
   s->ty = ty;
   s->H = H;
   s->hist = hist;
+  s->auto_launch = false;
   return IDMX_OK;
 }
 

@@ -315,6 +315,26 @@ struct Impl {
     }
   }
 
+  // One step of a small 3D lattice (k_tile3d).
+  static hipError_t tile3(idmx_sc_s* s, const T* pop, T* swap, double* n, double* psi, double* u) {
+    if constexpr (S::D == 3) {
+      using SH = Tile3Shape<ES>;
+      const Geom& g = s->geo;
+      const int ntx = (g.L0 + SH::TX - 1) / SH::TX, nty = (g.L1 + SH::TY - 1) / SH::TY;
+      const int ntiles = ntx * nty * ((g.L2 + SH::TZ - 1) / SH::TZ);
+      const unsigned grid = (unsigned)((ntiles + 7) / 8 * 8);
+      if (n)
+        hipLaunchKernelGGL((k_tile3d<ES, T, SHIFT, COLL, true>), dim3(grid), dim3(SH::NT), 0,
+                           s->ctx->stream, pop, swap, g, phys(s), ntx, nty, ntiles, n, psi, u);
+      else
+        hipLaunchKernelGGL((k_tile3d<ES, T, SHIFT, COLL, false>), dim3(grid), dim3(SH::NT), 0,
+                           s->ctx->stream, pop, swap, g, phys(s), ntx, nty, ntiles, n, psi, u);
+      return hipGetLastError();
+    } else {
+      return hipErrorInvalidConfiguration;
+    }
+  }
+
   // Tile shapes the autotuner chooses from; the step that writes n/psi/u at
   // a checkpoint uses one fixed shape.
   template <bool WF>
@@ -433,7 +453,11 @@ struct Impl {
     // (small 2D lattices with the E4 force stay on the streamed storage on
     // variant 10: kTileSteps steps per launch, single steps with registers)
     const bool small = kTile && !fwalls && s->geo.V < kPairSites;
-    const bool xs = fwalls || (COLL < 3 ? s->hist == 10 && !small : (kFixedDma2 || kFixedDma3));
+    // small 3D lattices, unless a launch was set: k_tile3d
+    const bool small3 = S::D == 3 && !twop && !fwalls && s->auto_launch &&
+                        s->geo.V < (sizeof(T) == 4 ? kTile3Sites32 : kTile3Sites);
+    const bool xs = !small3 && (fwalls || (COLL < 3 ? s->hist == 10 && !small
+                                                    : (kFixedDma2 || kFixedDma3)));
     const int nxsh = xs && !twop ? nsteps - (wf ? 1 : 0) : 0;
     if constexpr (COLL < 3) if (pull) {
       hipLaunchKernelGGL((k_restream<S, T>), dim3(grid_for(s->geo.V)), dim3(256), 0, st,
@@ -489,7 +513,10 @@ struct Impl {
       hipError_t e;
       if (pev) IDMX_HIP(hipEventRecord(pev[2 * k], st));
       hipEvent_t mid = pev ? pev[2 * k + 1] : nullptr;
-      if constexpr (COLL >= 3) {
+      if (small3) {
+        if (mid) IDMX_HIP(hipEventRecord(mid, st));
+        e = tile3(s, a, b, wf && last ? n : nullptr, psi, u);
+      } else if constexpr (COLL >= 3) {
         // the Shan-Chen forcing and the isotropy filter: the fixed fused
         // launch, or the two-pass step (walls, a body force, a psi program,
         // IDMX_RUN_TWO_PASS)

@@ -535,6 +535,31 @@ __device__ __forceinline__ void st_nt_sbase(uint64_t base, uint32_t off, T v) {
   __builtin_nontemporal_store(v, (IDMX_GLOBAL T*)(b + off));
 }
 
+// Makes the Q loaded values of a site all known at one point. Summed as they
+// are loaded, they cost a memory latency each: to save registers the compiler
+// puts every load right before its addition.
+template <class T>
+__device__ __forceinline__ void arrive(T (&f)[9]) {
+  asm volatile("" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]),
+               "+v"(f[6]), "+v"(f[7]), "+v"(f[8]));
+}
+template <class T>
+__device__ __forceinline__ void arrive(T (&f)[19]) {
+  asm volatile("" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]),
+               "+v"(f[6]), "+v"(f[7]), "+v"(f[8]), "+v"(f[9]), "+v"(f[10]), "+v"(f[11]),
+               "+v"(f[12]), "+v"(f[13]), "+v"(f[14]), "+v"(f[15]), "+v"(f[16]), "+v"(f[17]),
+               "+v"(f[18]));
+}
+
+// Sum of a site's populations, in order.
+template <int Q, class T>
+__device__ __forceinline__ T pop_sum(const T (&f)[Q]) {
+  T s = f[0];
+#pragma unroll
+  for (int q = 1; q < Q; q++) s += f[q];
+  return s;
+}
+
 // Push-stream one site's f* to its neighbours (periodic).
 template <class S, class T>
 __device__ inline void push_store(T* __restrict__ dst, const Geom& geo, int x,

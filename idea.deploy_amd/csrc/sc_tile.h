@@ -1,5 +1,6 @@
-// sc_tile.h -- four time steps of a small D2Q9 lattice (E4 force) in one
-// launch.
+// sc_tile.h -- steps of small lattices: four time steps of a D2Q9 lattice (E4
+// force) in one launch (k_tile2d), one step of a D3Q19 lattice without a
+// march (k_tile3d).
 //
 // What bounds a small lattice is latency: a step of 128^2 sites moves 2.4 MB
 // that stay in L2 and is over in 5.2 us, most of it launch, two memory
@@ -113,6 +114,136 @@ k_tile2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
   stage(std::integral_constant<int, 1>{}, fa[0], SH::F0, fb[0], SH::F1, pb);
   stage(std::integral_constant<int, 2>{}, fb[0], SH::F1, fa[0], SH::F0, pa);
   stage(std::integral_constant<int, 3>{}, fa[0], SH::F0, nullptr, 0, pb);
+}
+
+// --------------------------------------------------------------------------
+// One step of a small D3Q19 lattice, one site per thread: a block loads a
+// 16 x 4 x 4 tile and sums the densities of its R-wide halo, all loads
+// independent of each other, then collides and pushes. The march of
+// k_fused / k_fused_dma reads each population about once, but as a chain of
+// H + 2R dependent planes, and a lattice of 10^4 to 10^5 sites leaves no
+// second block on a CU to hide them; this step reads 2.5 times the sites
+// (R = 1), from L2, in one round trip. Bound by that round trip and the launch
+// on 24^3 (7.6 us per step, the march 13.1), by L2 traffic on 48 x 44 x 40
+// (E4 FP64 11.6 against 14.1, dense MRT 20.4 against 32.6). 16 x 4 x 4: one
+// wave per z plane, four whole 128-byte lines of FP64 per row load.
+template <class ES>
+struct Tile3Shape {
+  static constexpr int R = ES::R, TX = 16, TY = 4, TZ = 4, NT = TX * TY * TZ;
+  static constexpr int PX = TX + 2 * R, PY = TY + 2 * R, PZ = TZ + 2 * R;
+  static constexpr int SLAB = 2 * R * PX * PY;          // halo sites of the z slabs
+  static constexpr int RING = PX * PY - TX * TY;        // of each plane between them
+  static constexpr int NH = SLAB + TZ * RING;
+  static constexpr int YS = 2 * R * PX;                 // of a ring's y slabs
+};
+
+template <class ES, class T, bool SHIFT, int COLL, bool WF>
+__global__ void __launch_bounds__(256)
+k_tile3d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> P, int ntx,
+         int nty, int ntiles, double* __restrict__ n_out, double* __restrict__ psi_out,
+         double* __restrict__ u_out) {
+  using S = D3Q19;
+  using SH = Tile3Shape<ES>;
+  constexpr int Q = S::Q, R = SH::R, PX = SH::PX, PY = SH::PY, NB = NBasis<3>::value;
+  constexpr int NTAB = COLL == 2 ? Q : COLL == 1 ? Q * Q + 2 * NB * Q : 1;
+  __shared__ T psi[SH::PZ][PY][PX];
+  __shared__ T tab[NTAB];
+  const int per = gridDim.x >> 3;
+  int t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (t >= ntiles) return;
+  const int x0 = t % ntx * SH::TX;
+  t /= ntx;
+  const int y0 = t % nty * SH::TY, z0 = t / nty * SH::TZ;
+  const int tid = threadIdx.x;
+  Phys<T> PL = P;
+  if constexpr (COLL == 1 || COLL == 2) {
+    for (int i = tid; i < NTAB; i += SH::NT) tab[i] = P.mrtA[i];
+    PL.mrtA = tab;
+    PL.mrtB = COLL == 1 ? tab + Q * Q : nullptr;
+    PL.mrtG = COLL == 1 ? tab + Q * Q + NB * Q : nullptr;
+  }
+  // periodic coordinate, one period out of range at most where the axis is as
+  // long as the haloed tile
+  auto per1 = [](int v, int L) {
+    if (L >= PX) return wrap(v, L);
+    return ((v % L) + L) % L;
+  };
+  const int tx = tid % SH::TX, ty = tid / SH::TX % SH::TY;
+  const int tz = __builtin_amdgcn_readfirstlane(tid / (SH::TX * SH::TY));  // one plane per wave
+  const int x = x0 + tx, y = y0 + ty, z = z0 + tz;
+  const bool own = x < geo.L0 && y < geo.L1 && z < geo.L2;
+  const int xw = per1(x, geo.L0), yw = per1(y, geo.L1), zw = per1(z, geo.L2);
+  const uint32_t E = (uint32_t)sizeof(T), L0 = (uint32_t)geo.L0, L01 = L0 * (uint32_t)geo.L1;
+  const uint64_t qbytes = (uint64_t)geo.V * sizeof(T);
+  auto load = [&](uint64_t base, uint32_t off, T (&f)[Q]) {
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      f[q] = *(const IDMX_GLOBAL T*)((const IDMX_GLOBAL char*)sgpr_u64(base) + off);
+      base += qbytes;
+    }
+  };
+  T f[Q];
+  const uint32_t own_off = ((uint32_t)xw + L0 * (uint32_t)yw) * E;
+  load((uint64_t)pop + (uint64_t)L01 * (uint32_t)zw * E, own_off, f);
+#pragma unroll
+  for (int k = 0; k < (SH::NH + SH::NT - 1) / SH::NT; k++) {
+    const int h = tid + k * SH::NT;
+    if (h < SH::NH) {
+      int hx, hy, hz;
+      if (h < SH::SLAB) {
+        const int p = h / (PX * PY), r = h % (PX * PY);
+        hz = p < R ? p : SH::TZ + p;
+        hy = r / PX;
+        hx = r % PX;
+      } else {
+        const int k2 = h - SH::SLAB, r = k2 % SH::RING;
+        hz = R + k2 / SH::RING;
+        if (r < SH::YS) {
+          const int p = r / PX;
+          hy = p < R ? p : SH::TY + p;
+          hx = r % PX;
+        } else {
+          const int c = (r - SH::YS) % (2 * R);
+          hy = R + (r - SH::YS) / (2 * R);
+          hx = c < R ? c : SH::TX + c;
+        }
+      }
+      const uint32_t off = ((uint32_t)per1(x0 - R + hx, geo.L0) +
+                            L0 * (uint32_t)per1(y0 - R + hy, geo.L1) +
+                            L01 * (uint32_t)per1(z0 - R + hz, geo.L2)) * E;
+      T fh[Q];
+      load((uint64_t)pop, off, fh);
+      arrive(fh);
+      const T s = pop_sum(fh);
+      psi[hz][hy][hx] = psi_of(P.psi_kind, SHIFT ? P.rho0 + s : s);
+    }
+  }
+  const T dn = pop_sum(f);
+  const T lpsi = psi_of(P.psi_kind, SHIFT ? P.rho0 + dn : dn);
+  psi[tz + R][ty + R][tx + R] = lpsi;
+  __syncthreads();
+  if (!own) return;
+  T gx, gy, gz, fo[Q], u[3];
+  iso_grad<ES>(
+      [&](int e) { return psi[tz + R + ES::ez[e]][ty + R + ES::ey[e]][tx + R + ES::ex[e]]; }, gx,
+      gy, gz);
+  collide<S, T, SHIFT, COLL>(f, dn, gx, gy, gz, lpsi, PL, fo, u);
+  // push: in-plane offsets per lane, the target plane in the scalar base
+  const int xs[3] = {wrap(x - 1, geo.L0), x, wrap(x + 1, geo.L0)};
+  const int ys[3] = {wrap(y - 1, geo.L1), y, wrap(y + 1, geo.L1)};
+  const int zs[3] = {wrap(z - 1, geo.L2), z, wrap(z + 1, geo.L2)};
+#pragma unroll
+  for (int q = 0; q < Q; q++)
+    st_nt_sbase((uint64_t)pop_swap + q * qbytes + (uint64_t)L01 * (uint32_t)zs[S::cz[q] + 1] * E,
+                ((uint32_t)xs[S::cx[q] + 1] + L0 * (uint32_t)ys[S::cy[q] + 1]) * E, fo[q]);
+  if (WF) {
+    const int64_t g = lex(geo, x, y, z);
+    n_out[g] = (double)(SHIFT ? P.rho0 + dn : dn);
+    psi_out[g] = (double)lpsi;
+    u_out[g] = (double)u[0];
+    u_out[g + geo.V] = (double)u[1];
+    u_out[g + 2 * geo.V] = (double)u[2];
+  }
 }
 
 }  // namespace idmx

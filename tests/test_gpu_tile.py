@@ -4,7 +4,9 @@ in registers (variant 1), or against the two-pass step for the Shan-Chen
 forcing and the isotropy filter: the same arithmetic per site, equal in FP64
 and, contraction being the same in every launch, to rounding in FP32. Lattices
 smaller than a tile and its ring, edges of the 8 x 8 and 16 x 16 tiles, and
-runs that leave single steps over."""
+runs that leave single steps over. Likewise one step of a small 3D lattice
+without a march (k_tile3d), on lattices shorter than its 16 x 4 x 4 tile and
+its halo and ones that leave partial tiles."""
 import numpy as np
 import pytest
 
@@ -65,3 +67,51 @@ def test_four_steps_per_launch_equal_single_steps(tenet, dims, prec, coll, steps
         else:
             # ~10 roundings of 6e-8 of the largest value per step
             assert np.abs(r - g).max() <= steps * 10 * 6e-8 * np.abs(r).max()
+
+
+CASES3 = [('D3E4', (3, 3, 3), 'fp64', 'bgk'), ('D3E8', (5, 5, 5), 'fp64', 'mrt'),
+          ('D3E4', (17, 5, 9), 'fp64', 'mrt'), ('D3E4', (48, 44, 40), 'fp64', 'mrt'),
+          ('D3E6', (31, 9, 6), 'fp64', 'bgk'), ('D3E8', (33, 29, 31), 'fp64', 'bgk'),
+          ('D3E4', (18, 6, 40), 'fp64', 'dense'), ('D3E4', (16, 70, 5), 'fp64', 'sc'),
+          ('D3E4', (40, 41, 42), 'fp32s', 'mrt'), ('D3E8', (21, 22, 23), 'fp32s', 'bgk')]
+
+
+@pytest.mark.parametrize('es,dims,prec,coll', CASES3)
+@pytest.mark.parametrize('wf', [True, False])
+def test_small_3d_step_equals_march(tenet, es, dims, prec, coll, wf):
+    from idmx.IdpyCode import IdpyMemory
+    from idmx.LBM import hermite
+    from idmx.LBM._base import PopArray
+    from idmx.LBM._engine import SCEngine
+    S = np.diag(np.linspace(0.7, 1.5, 19))
+    if coll == 'dense':
+        S[5, 6] = 0.05
+    kw = {'mrt': hermite.mrt_kernel_tables('D3Q19', S)} if coll in ('mrt', 'dense') else \
+        {'forcing': 'sc'} if coll == 'sc' else {}
+    V = int(np.prod(dims))
+    n0 = 1.0 + 0.3 * np.sin(2 * np.pi * np.arange(V) / 17 + 0.3)
+    out = []
+    for march in (False, True):
+        eng = SCEngine(tenet, 'D3Q19', es, dims, 'exp', -5.0 / 3.0, 1.0, precision=prec,
+                       rho0=1.0, **kw)
+        if march:
+            eng.set_launch(32, 8, 2, 1)
+        n = IdpyMemory.OnDevice(n0, tenet)
+        psi = IdpyMemory.Zeros(V, np.float64, tenet)
+        u = IdpyMemory.Zeros(3 * V, np.float64, tenet)
+        a, b = PopArray(eng, tenet), PopArray(eng, tenet)
+        eng.init_pop(a, n, u)
+        swapped = eng.run(a, b, 5, n=n, psi=psi, u=u, write_fields=wf,
+                          two_pass=march and coll == 'sc')
+        out.append([(b if swapped else a).RawD2H()]
+                   + ([n.D2H(), psi.D2H()] + ([u.D2H()] if prec == 'fp64' else []) if wf else []))
+        for x in (a, b, n, psi, u):
+            x.Free()
+        eng.close()
+    for g, r in zip(*out):
+        assert np.isfinite(g).all()
+        if prec == 'fp64':
+            assert np.array_equal(r, g)
+        else:
+            # ~10 roundings of 6e-8 of the largest value per step
+            assert np.abs(r - g).max() <= 5 * 10 * 6e-8 * np.abs(r).max()
