@@ -241,18 +241,21 @@ struct Impl {
   // per step against 10.8 with single steps, 256^2 9.5 against 6.4 (1024^2
   // MRT: 21.8 against 38.6). A lattice much narrower than a block leaves its
   // lanes idle.
-  static PairPlan pair_plan(const idmx_sc_s* s) {
+  // With walls (1024 x 768: 20.3 us per step, single steps 34.6) 128 threads
+  // where both cost the same (256: 23.6, its waves longer in each other's
+  // barrier; 700 x 900 18.9 and 20.0).
+  static PairPlan pair_plan(const idmx_sc_s* s, bool walls) {
     PairPlan p;
     if constexpr (S::D == 2)
       if (s->geo.V >= kPairSites) {
-        const double c = pair_cost<256>(s->geo, p, 1e300);
-        pair_cost<128>(s->geo, p, c);
+        if (walls) pair_cost<256>(s->geo, p, pair_cost<128>(s->geo, p, 1e300));
+        else pair_cost<128>(s->geo, p, pair_cost<256>(s->geo, p, 1e300));
         const int ntx = (s->geo.L0 + p.txo - 1) / p.txo;
         if (2 * s->geo.L0 < ntx * p.nt) p.nt = 0;
       }
     return p;
   }
-  template <int NT, bool WF>
+  template <int NT, bool WF, bool WALLS = false>
   static hipError_t launch_pair(idmx_sc_s* s, const PairPlan& p, const T* pop, T* swap, double* n,
                                 double* psi, double* u) {
     if constexpr (S::D == 2) {
@@ -260,16 +263,24 @@ struct Impl {
       const int ntx = (g.L0 + p.txo - 1) / p.txo, H = std::min(p.H, g.L1);
       const int ntiles = ntx * ((g.L1 + H - 1) / H);
       const unsigned grid = (unsigned)((ntiles + 7) / 8 * 8);
-      hipLaunchKernelGGL((k_pair2d<ES, T, SHIFT, COLL, NT, WF>), dim3(grid), dim3(NT), 0,
+      hipLaunchKernelGGL((k_pair2d<ES, T, SHIFT, COLL, NT, WF, WALLS>), dim3(grid), dim3(NT), 0,
                          s->ctx->stream, pop, swap, g, phys(s), p.txo, H, ntx, ntiles, s->xsh, n,
-                         psi, u);
+                         psi, u, (const uint64_t*)s->wmask_dev, (T)s->bforce[0], (T)s->bforce[1]);
       return hipGetLastError();
     } else {
       return hipErrorInvalidConfiguration;
     }
   }
-  static hipError_t pair(idmx_sc_s* s, const PairPlan& p, const T* pop, T* swap, double* n,
-                         double* psi, double* u) {
+  static hipError_t pair(idmx_sc_s* s, const PairPlan& p, bool walls, const T* pop, T* swap,
+                         double* n, double* psi, double* u) {
+    if constexpr (kFusedWalls)
+      if (walls) {
+        if (p.nt == 128)
+          return n ? launch_pair<128, true, true>(s, p, pop, swap, n, psi, u)
+                   : launch_pair<128, false, true>(s, p, pop, swap, n, psi, u);
+        return n ? launch_pair<256, true, true>(s, p, pop, swap, n, psi, u)
+                 : launch_pair<256, false, true>(s, p, pop, swap, n, psi, u);
+      }
     if (p.nt == 128)
       return n ? launch_pair<128, true>(s, p, pop, swap, n, psi, u)
                : launch_pair<128, false>(s, p, pop, swap, n, psi, u);
@@ -467,7 +478,7 @@ struct Impl {
     }
     // two steps per launch: an even number of pairs, so that the state ends in
     // the buffer in which single steps would leave it
-    const PairPlan pp = S::D == 2 && xs && !twop && !fwalls && !pev ? pair_plan(s) : PairPlan{};
+    const PairPlan pp = S::D == 2 && xs && !twop && !pev ? pair_plan(s, fwalls) : PairPlan{};
     const int npair = pp.nt ? nsteps / 2 & ~1 : 0;
     if (npair > 0) {
       const int nl = nsteps - npair;  // single steps first, then the pairs
@@ -477,7 +488,8 @@ struct Impl {
         s->xsh = (k > 0 ? 1 : 0) | (k < nl - 1 ? 2 : 0);
         const bool f = wf && k == nl - 1;
         hipError_t e;
-        if (k >= nl - npair) e = pair(s, pp, a, b, f ? n : nullptr, psi, u);
+        if (k >= nl - npair) e = pair(s, pp, fwalls, a, b, f ? n : nullptr, psi, u);
+        else if (fwalls) e = fused_walls(s, a, b, psi);
         else if constexpr (COLL >= 3) e = fused_fixed<false>(s, a, b, nullptr, nullptr, nullptr);
         else e = fused<false>(s, a, b, nullptr, nullptr, nullptr);
         s->xsh = 0;

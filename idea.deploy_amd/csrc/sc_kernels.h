@@ -1012,11 +1012,12 @@ struct DmaShape {
       LDS <= 160 * 1024 && NT % 64 == 0 && (!WALLS || sizeof(T) == sizeof(double));
 };
 
-// Wall mask of a site for the fused step with walls: bit q (q >= 1) when the
+// Wall mask of a site for the fused steps with walls: bit q (q >= 1) when the
 // neighbour x + c_q is solid (flag 0: the population pushed there bounces
-// back), bit 63 when the site itself is not fluid (flag != 1: not updated,
-// its psi is the one the caller stored).
-constexpr int kWallSelf = 63;
+// back), bit 0 when the site itself is not fluid (flag != 1: not updated, its
+// psi is the one the caller stored), bit Q + q when the neighbour x - c_q is
+// neither (nothing streams in from there).
+constexpr int kWallSelf = 0;
 
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -1430,7 +1431,9 @@ k_wall_mask(const uint8_t* __restrict__ walls, Geom geo, uint64_t* __restrict__ 
       const int xt = S::cx[q] ? wrap(x + S::cx[q], geo.L0) : x;
       const int yt = S::cy[q] ? wrap(y + S::cy[q], geo.L1) : y;
       const int zt = S::cz[q] ? wrap(z + S::cz[q], geo.L2) : z;
-      if (walls[lex(geo, xt, yt, zt)] == 0) m |= uint64_t(1) << q;
+      const uint8_t w = walls[lex(geo, xt, yt, zt)];
+      if (w == 0) m |= uint64_t(1) << q;
+      else if (w != 1) m |= uint64_t(1) << (S::Q + opposite<S>(q));
     }
     mask[g] = m;
   }

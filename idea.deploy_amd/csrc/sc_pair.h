@@ -33,7 +33,7 @@
 
 namespace idmx {
 
-template <class ES, class T, int COLL, int NT>
+template <class ES, class T, int COLL, int NT, bool WALLS = false>
 struct PairShape {
   static constexpr int R = ES::R;
   static constexpr int HALO = 2 * R + 1;  // columns (rows) of f(0) beyond the written ones
@@ -42,8 +42,10 @@ struct PairShape {
   static constexpr int PX = NT + 2 * R;   // row of psi
   static constexpr int NS = 2 * R + 1;    // psi ring rows
   // rows kept of f*(0) by c_qy: +1 three, 0 two, -1 one (the rest population
-  // stays in registers)
-  static constexpr int FROWS = 3 * 3 + 2 * 2 + 3 * 1;
+  // stays in registers); with walls -1 two, since a population that bounces
+  // back is staged one row above the pushed ones
+  static constexpr int DOWN = WALLS ? 2 : 1;
+  static constexpr int FROWS = 3 * 3 + 2 * 2 + 3 * DOWN;
   static constexpr int NB = NBasis<2>::value;
   static constexpr int Q = D2Q9::Q;
   static constexpr int NTAB = COLL == 2 ? Q : COLL == 1 ? Q * Q + 2 * NB * Q : 1;
@@ -53,13 +55,17 @@ struct PairShape {
 // k_fused_dma (bit 0: reads the x-shifted storage, bit 1: writes it); WF: the
 // second step also writes n, psi and u. Compiled for two waves per SIMD: at
 // three the E4 step spills and runs at 296 us (4096^2) instead of 286.
-template <class ES, class T, bool SHIFT, int COLL, int NT, bool WF>
+// WALLS: as in k_fused_dma; psi_out holds the psi of the solid sites, which
+// stays, wmask the masks.
+template <class ES, class T, bool SHIFT, int COLL, int NT, bool WF, bool WALLS = false>
 __global__ void __launch_bounds__(NT, 2)
 k_pair2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> P, int txo,
          int H, int ntx, int ntiles, int xsh, double* __restrict__ n_out,
-         double* __restrict__ psi_out, double* __restrict__ u_out) {
+         double* psi_out, double* __restrict__ u_out, const uint64_t* __restrict__ wmask = nullptr,
+         T bx = T(0), T by = T(0)) {
   using S = D2Q9;
-  using SH = PairShape<ES, T, COLL, NT>;
+  using SH = PairShape<ES, T, COLL, NT, WALLS>;
+  static_assert(!WALLS || (ES::R == 1 && sizeof(T) == 8 && !SHIFT));
   constexpr int Q = S::Q, R = ES::R, HALO = SH::HALO, NS = SH::NS;
   __shared__ T frow[SH::FROWS][SH::FX];
   __shared__ T ring0[NS][SH::PX], ring1[NS][SH::PX];
@@ -94,7 +100,7 @@ k_pair2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
   // first staged row of population q
   auto f_base = [](int q) constexpr {
     int b = 0;
-    for (int k = 1; k < q; k++) b += S::cy[k] > 0 ? 3 : S::cy[k] < 0 ? 1 : 2;
+    for (int k = 1; k < q; k++) b += S::cy[k] > 0 ? 3 : S::cy[k] < 0 ? SH::DOWN : 2;
     return b;
   };
   const uint64_t qbytes = (uint64_t)geo.V * sizeof(T), rbytes = (uint64_t)geo.L0 * sizeof(T);
@@ -102,8 +108,17 @@ k_pair2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
   // rows of the lattice: `lrow` the next one to load, `srow` the next one to
   // store, stepped instead of reduced modulo L1 in every iteration
   int lrow = ((m0 - HALO) % Lm + Lm) % Lm, srow = m0;
+  // masks of rows j to j - 4 and, in flight with fn, of the next; its psi
+  uint32_t mn = 0, mk[5] = {};
+  double pn = 0;
   auto load_row = [&](T (&f)[Q]) {
     uint64_t base = (uint64_t)pop + (uint64_t)lrow * rbytes;
+    if constexpr (WALLS) {
+      mn = *(const IDMX_GLOBAL uint32_t*)((const IDMX_GLOBAL char*)sgpr_u64(
+                                              (uint64_t)wmask + (uint64_t)lrow * rbytes) + l0);
+      pn = *(const IDMX_GLOBAL double*)((const IDMX_GLOBAL char*)sgpr_u64(
+                                            (uint64_t)psi_out + (uint64_t)lrow * rbytes) + l0);
+    }
     lrow = lrow + 1 == Lm ? 0 : lrow + 1;
 #pragma unroll
     for (int q = 0; q < Q; q++) {
@@ -135,18 +150,27 @@ k_pair2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
     constexpr int B1 = (A1 + 1) % HR;        // row j - 2R - 2
     auto pslot = [&](int d) { return ps + d < 0 ? ps + d + NS : ps + d; };  // row j + d, d <= 0
     auto slot = [&](int q, int d) {  // f*(0) row j + d of population q, -6 <= d <= 0
-      if (S::cy[q] < 0) return 0;
+      if (S::cy[q] < 0 && SH::DOWN == 1) return 0;
       const int n = S::cy[q] > 0 ? 3 : 2;
       const int v = (S::cy[q] > 0 ? j3 : j2) + (d + 3 * n) % n;
       return v >= n ? v - n : v;
     };
+    // psi of row j - R - 2 where that is a solid site
+    T psolid = T(0);
+    if constexpr (WALLS) {
+      psolid = ring0[ps][tid + R];
+#pragma unroll
+      for (int k = 4; k > 0; k--) mk[k] = mk[k - 1];
+      mk[0] = mn;
+    }
     // psi(0) of row j
     if (j < J - 1) {
+      const T pw = pn;
 #pragma unroll
       for (int q = 0; q < Q; q++) fh0[A0][q] = fn[q];
       dn0[A0] = sum(fh0[A0]);
       if (j + 1 < J - 1) load_row(fn);
-      ring0[ps][tid + R] = psi_at(dn0[A0]);
+      ring0[ps][tid + R] = WALLS && (mk[0] & (1u << kWallSelf)) ? pw : psi_at(dn0[A0]);
     }
     // f(1) and psi(1) of row j - R - 2
     if (j >= 2 * R + 3) {
@@ -154,7 +178,7 @@ k_pair2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
       for (int q = 0; q < Q; q++)
         fh1[A1][q] = q == 0 ? rest0 : frow[f_base(q) + slot(q, -R - 2)][tid + 1];
       dn1[A1] = sum(fh1[A1]);
-      ring1[ps][tid + R] = psi_at(dn1[A1]);
+      ring1[ps][tid + R] = WALLS && (mk[3] & (1u << kWallSelf)) ? psolid : psi_at(dn1[A1]);
     }
     lds_barrier();
     rest0 = rest1;
@@ -163,12 +187,28 @@ k_pair2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
       T gx_, gy_, gz_, fo[Q], u[3];
       iso_grad<ES>([&](int e) { return ring0[pslot(ES::ey[e] - R)][tid + R + ES::ex[e]]; }, gx_,
                    gy_, gz_);
-      collide<S, T, SHIFT, COLL>(fh0[B0], dn0[B0], gx_, gy_, T(0), ring0[pslot(-R)][tid + R], PL,
-                                 fo, u);
+      collide<S, T, SHIFT, COLL, WALLS>(fh0[B0], dn0[B0], gx_, gy_, T(0),
+                                        ring0[pslot(-R)][tid + R], PL, fo, u, bx, by);
       rest1 = fo[0];
+      // with walls, most waves have no solid site near: one test for the wave
+      const uint32_t m = mk[1];
+      if (WALLS && __ballot(m != 0) != 0) {
+        if (!(m & (1u << kWallSelf))) {
 #pragma unroll
-      for (int q = 1; q < Q; q++)
-        frow[f_base(q) + slot(q, S::cy[q] - R)][tid + 1 + S::cx[q]] = fo[q];
+          for (int q = 1; q < Q; q++) {
+            // aimed at a solid site: back to this one as the opposite
+            const int o = opposite<S>(q);
+            if (m >> q & 1) frow[f_base(o) + slot(o, -R)][tid + 1] = fo[q];
+            else frow[f_base(q) + slot(q, S::cy[q] - R)][tid + 1 + S::cx[q]] = fo[q];
+            // a population that nothing streams into keeps its value
+            if (m >> (Q + q) & 1) frow[f_base(q) + slot(q, -R)][tid + 1] = fh0[B0][q];
+          }
+        }
+      } else {
+#pragma unroll
+        for (int q = 1; q < Q; q++)
+          frow[f_base(q) + slot(q, S::cy[q] - R)][tid + 1 + S::cx[q]] = fo[q];
+      }
     }
     // second step's collision of row j - 2R - 2 (psi(1) of row j - R - 2 + d
     // is in the slot of psi(0) row j + d)
@@ -177,14 +217,32 @@ k_pair2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
       iso_grad<ES>([&](int e) { return ring1[pslot(ES::ey[e] - R)][tid + R + ES::ex[e]]; }, gx_,
                    gy_, gz_);
       const T lpsi = ring1[pslot(-R)][tid + R];
-      collide<S, T, SHIFT, COLL>(fh1[B1], dn1[B1], gx_, gy_, T(0), lpsi, PL, fo, u);
-      if (own) {
+      collide<S, T, SHIFT, COLL, WALLS>(fh1[B1], dn1[B1], gx_, gy_, T(0), lpsi, PL, fo, u, bx,
+                                        by);
+      if (own && !(WALLS && (mk[4] & (1u << kWallSelf)))) {
         const int sup = srow + 1 == Lm ? 0 : srow + 1, sdn = srow == 0 ? Lm - 1 : srow - 1;
-#pragma unroll
-        for (int q = 0; q < Q; q++)
+        auto push = [&](int q) {
           st_nt_sbase((uint64_t)pop_swap + q * qbytes +
                           (uint64_t)(S::cy[q] > 0 ? sup : S::cy[q] < 0 ? sdn : srow) * rbytes,
                       S::cx[q] > 0 ? sp : S::cx[q] < 0 ? sm : l0, fo[q]);
+        };
+        if (WALLS && __ballot(mk[4] != 0) != 0) {
+#pragma unroll
+          for (int q = 0; q < Q; q++) {
+            // back to this site as the opposite: in the x-shifted storage
+            // that is kept at x - c_x of the opposite
+            if (q > 0 && (mk[4] >> q & 1))
+              st_nt_sbase((uint64_t)pop_swap + opposite<S>(q) * qbytes + (uint64_t)srow * rbytes,
+                          S::cx[q] == 0 || !wsh
+                              ? l0
+                              : (uint32_t)wrap(gx + S::cx[q], geo.L0) * (uint32_t)sizeof(T),
+                          fo[q]);
+            else push(q);
+          }
+        } else {
+#pragma unroll
+          for (int q = 0; q < Q; q++) push(q);
+        }
         if (WF) {
           const int64_t g = (int64_t)gx + (int64_t)geo.L0 * srow;
           n_out[g] = (double)(SHIFT ? P.rho0 + dn1[B1] : dn1[B1]);

@@ -9,7 +9,7 @@ single steps, and 3 steps none."""
 import numpy as np
 import pytest
 
-from helpers import droplet_field
+from helpers import droplet_field, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -66,3 +66,51 @@ def test_two_steps_per_launch_equal_single_steps(tenet, es, dims, prec, coll, st
         else:
             # ~10 roundings of 6e-8 of the largest value per step
             assert np.abs(r - g).max() <= steps * 10 * 6e-8 * np.abs(r).max()
+
+
+@pytest.mark.parametrize('dims,g', [((1024, 520), 1e-5), ((613, 643), 0.0), ((251, 1571), 2e-5)])
+@pytest.mark.parametrize('steps,wf', [(3, True), (4, True), (5, False), (8, True), (11, False)])
+def test_two_steps_per_launch_with_walls(tenet, dims, g, steps, wf):
+    """The walls step (plates, blocks across the periodic edges, lone solid
+    and lone fluid sites) against the two-pass step on the fluid sites: the
+    same arithmetic in the same order."""
+    from idmx.IdpyCode import IdpyMemory
+    from idmx.LBM._base import PopArray
+    from idmx.LBM._engine import SCEngine
+    rng = np.random.default_rng(5)
+    w = np.ones(dims[::-1], dtype=np.uint8)
+    w[0] = w[-1] = 0
+    w[dims[1] // 3:dims[1] // 3 + 5, :3] = 0
+    w[dims[1] // 3:dims[1] // 3 + 5, -2:] = 0
+    w[dims[1] // 2:dims[1] // 2 + 40, dims[0] // 2:dims[0] // 2 + 60] = 0
+    w[dims[1] // 2 + 7, dims[0] // 2 + 9] = 1
+    w[rng.integers(0, dims[1], 4000), rng.integers(0, dims[0], 4000)] = 0
+    psi_w = np.where(w == 0, rng.uniform(0.3, 0.7, size=w.shape), 0.0).ravel()
+    w = w.ravel()
+    fl, V, n0 = w == 1, w.size, droplet_field(dims, seed=8)
+    wd = IdpyMemory.OnDevice(w, tenet)
+    out = []
+    for two_pass in (True, False):
+        eng = SCEngine(tenet, 'D2Q9', 'D2E4', dims, 'exp', -5.0 / 3.0, 1.0)
+        eng.set_walls(wd)
+        if g:
+            eng.set_body_force(0.0, g, 0.0)
+        n = IdpyMemory.OnDevice(n0, tenet)
+        psi = IdpyMemory.OnDevice(psi_w, tenet)
+        u = IdpyMemory.Zeros(2 * V, np.float64, tenet)
+        a, b = PopArray(eng, tenet), PopArray(eng, tenet)
+        eng.init_pop(a, n, u)
+        swapped = eng.run(a, b, steps, n=n, psi=psi, u=u, write_fields=wf, two_pass=two_pass)
+        assert swapped == (steps % 2 == 1)
+        out.append((eng.pop_to_host_soa(b if swapped else a).reshape(9, V)[:, fl], n.D2H()[fl],
+                    psi.D2H(), u.D2H().reshape(2, V)[:, fl]))
+        for x in (n, psi, u, a, b):
+            x.Free()
+        eng.close()
+    wd.Free()
+    (f1, n1, p1, u1), (f2, n2, p2, u2) = out
+    assert np.isfinite(f2).all() and rel_err(f2.ravel(), f1.ravel()) <= 1e-15
+    assert np.array_equal(p2[~fl], psi_w[~fl])
+    if wf:
+        assert rel_err(n2, n1) <= 1e-15 and rel_err(p2[fl], p1[fl]) <= 1e-15
+        assert rel_err(u2.ravel(), u1.ravel()) <= 1e-14
