@@ -490,6 +490,7 @@ int idmx_sc_destroy(idmx_sc_t s) {
     hipStreamSynchronize(s->ctx->stream);
     if (s->psi_prog_dev) hipFree(s->psi_prog_dev);
     if (s->wmask_dev) hipFree(s->wmask_dev);
+    if (s->wflag_host) hipHostFree(s->wflag_host);
   }
   delete s;
   return IDMX_OK;
@@ -560,8 +561,10 @@ int idmx_sc_set_walls(idmx_sc_t s, const void* walls) {
   CHECK_ARG(s, "idmx_sc_set_walls: null simulation");
   // the per-site masks of the fused step with walls (FP64 BGK), allocated
   // here so that no run allocates
-  if (walls && !s->wmask_dev && s->pop_elem == 8 && s->coll == 0)
+  if (walls && !s->wmask_dev && s->pop_elem == 8 && s->coll == 0) {
+    if (!s->wflag_host) IDMX_HIP(hipHostMalloc(&s->wflag_host, sizeof(uint32_t), hipHostMallocMapped));
     IDMX_HIP(hipMalloc(&s->wmask_dev, sizeof(uint64_t) * (size_t)s->geo.V));
+  }
   s->walls = (const uint8_t*)walls;
   return IDMX_OK;
 }

@@ -301,22 +301,33 @@ struct Impl {
 
   // Four steps in one launch on a small 2D lattice (k_tile2d).
   static constexpr bool kTile = S::D == 2 && ES::R == 1;
-  template <int B, bool WF>
+  template <int B, bool WF, bool WALLS = false>
   static hipError_t launch_tile(idmx_sc_s* s, const T* pop, T* swap, double* n, double* psi,
                                 double* u) {
     const Geom& g = s->geo;
     const int ntx = (g.L0 + B - 1) / B, ntiles = ntx * ((g.L1 + B - 1) / B);
     const unsigned grid = (unsigned)((ntiles + 7) / 8 * 8);
-    hipLaunchKernelGGL((k_tile2d<T, SHIFT, COLL, B, kTileSteps, WF>), dim3(grid),
+    hipLaunchKernelGGL((k_tile2d<T, SHIFT, COLL, B, kTileSteps, WF, WALLS>), dim3(grid),
                        dim3(TileShape<B, kTileSteps>::NT), 0, s->ctx->stream, pop, swap, g,
-                       phys(s), ntx, ntiles, n, psi, u);
+                       phys(s), ntx, ntiles, n, psi, u, (const uint64_t*)s->wmask_dev,
+                       (T)s->bforce[0], (T)s->bforce[1]);
     return hipGetLastError();
   }
-  static hipError_t tile(idmx_sc_s* s, const T* pop, T* swap, double* n, double* psi, double* u) {
+  static hipError_t tile(idmx_sc_s* s, bool walls, const T* pop, T* swap, double* n, double* psi,
+                         double* u) {
     if constexpr (kTile) {
       // 8 x 8 tiles while every one has a CU of its own (128^2: 1.92 us per
       // step against 2.50), else 16 x 16 (256^2: 2.53 against 4.24)
-      if ((int64_t)((s->geo.L0 + 7) / 8) * ((s->geo.L1 + 7) / 8) <= 256)
+      const bool b8 = (int64_t)((s->geo.L0 + 7) / 8) * ((s->geo.L1 + 7) / 8) <= 256;
+      if constexpr (kFusedWalls)
+        if (walls) {
+          if (b8)
+            return n ? launch_tile<8, true, true>(s, pop, swap, n, psi, u)
+                     : launch_tile<8, false, true>(s, pop, swap, n, psi, u);
+          return n ? launch_tile<16, true, true>(s, pop, swap, n, psi, u)
+                   : launch_tile<16, false, true>(s, pop, swap, n, psi, u);
+        }
+      if (b8)
         return n ? launch_tile<8, true>(s, pop, swap, n, psi, u)
                  : launch_tile<8, false>(s, pop, swap, n, psi, u);
       return n ? launch_tile<16, true>(s, pop, swap, n, psi, u)
@@ -405,15 +416,15 @@ struct Impl {
     // with walls the step is the two-pass one (density and psi of the fluid
     // sites into n / psi, where psi also holds the solid sites' values)
     const bool body = s->bforce[0] != 0.0 || s->bforce[1] != 0.0 || s->bforce[2] != 0.0;
-    // walls (with or without a body force) run the fused step with walls; the
-    // step that writes n / psi / u at the end of a run is the two-pass one
-    // (from 2^19 sites up, or when asked for: on smaller lattices the
-    // two-pass step is as fast; measured 0.94x at 64^3, 1.07x at 1024^2,
+    // walls (with or without a body force) run the fused step with walls; a
+    // step of its own that writes n / psi / u is the two-pass one (from 2^19
+    // sites up, or when asked for: on smaller lattices two passes are as
+    // fast as single fused steps; measured 0.94x at 64^3, 1.07x at 1024^2,
     // 1.30x at 256^3 and 1.47x at 4096^2)
-    const bool fwalls = kFusedWalls && s->walls && (flags & IDMX_RUN_TWO_PASS) == 0 &&
+    bool fwalls = kFusedWalls && s->walls && (flags & IDMX_RUN_TWO_PASS) == 0 &&
                         s->desc.psi_kind != IDMX_PSI_PROGRAM &&
                         (s->geo.V >= (int64_t(1) << 19) || (flags & IDMX_RUN_FUSED_WALLS) != 0);
-    const bool twop = !fwalls && ((flags & IDMX_RUN_TWO_PASS) != 0 || s->walls || body ||
+    bool twop = !fwalls && ((flags & IDMX_RUN_TWO_PASS) != 0 || s->walls || body ||
                                   s->desc.psi_kind == IDMX_PSI_PROGRAM);
     if ((twop || fwalls) && (!n || !psi)) {
       set_error(s->walls || body || s->desc.psi_kind == IDMX_PSI_PROGRAM
@@ -447,9 +458,31 @@ struct Impl {
         return IDMX_E_NOMEM;
       }
       hipLaunchKernelGGL((k_wall_mask<S>), dim3(grid_for(s->geo.V)), dim3(256), 0, st, s->walls,
-                         s->geo, s->wmask_dev);
+                         s->geo, s->wmask_dev, (uint32_t*)nullptr);
       IDMX_HIP(hipGetLastError());
     }
+    // smaller 2D lattices with walls: several steps per launch, if every flag
+    // is 0 or 1 (waiting for that costs 10 us; a run of 8 steps of 128^2
+    // takes 45 us then, 69 on two passes). Two on the pair kernel where that
+    // applies (700 x 640 14.1 us per step; tiles 18.5, two passes 23.1), else
+    // kTileSteps on tiles (128^2 2.2 against 6.9, 256^2 2.9 against 8.0, 512^2
+    // 10.8 against 14.8, 150 x 2000 13.3 against 16.8). A run of two-pass
+    // steps leaves n and psi of its last step: so do the tiles, while the
+    // pairs are left to runs that ask for them.
+    bool wtile = false;
+    if constexpr (kTile && kFusedWalls)
+      if (twop && s->walls && (flags & IDMX_RUN_TWO_PASS) == 0 && !pev &&
+          s->desc.psi_kind != IDMX_PSI_PROGRAM && s->wmask_dev && nsteps >= 2 * kTileSteps) {
+        *s->wflag_host = 0;
+        hipLaunchKernelGGL((k_wall_mask<S>), dim3(grid_for(s->geo.V)), dim3(256), 0, st, s->walls,
+                           s->geo, s->wmask_dev, s->wflag_host);
+        IDMX_HIP(hipGetLastError());
+        IDMX_HIP(hipStreamSynchronize(st));
+        if (*s->wflag_host == 0) {
+          if (wf && pair_plan(s, true).nt) fwalls = true, twop = false;
+          else wtile = true;
+        }
+      }
     IDMX_HIP(hipEventRecord(s->ctx->ev0, st));
     // pull-form variants: convert the streamed populations to the pull form,
     // step in it, convert back (nsteps + 2 buffer swaps: same parity as
@@ -501,7 +534,7 @@ struct Impl {
     // reason; they and the single steps before them keep the streamed storage
     int nquad = 0;
     if constexpr (kTile)
-      if (small && !twop && !pev && (COLL >= 3 || s->hist == 10))
+      if (wtile || (small && !twop && !pev && (COLL >= 3 || s->hist == 10)))
         nquad = nsteps / kTileSteps & ~1;
     if constexpr (kTile)
       if (nquad > 0) {
@@ -509,11 +542,12 @@ struct Impl {
         for (int k = 0; k < nl; k++) {
           const T* a = (const T*)*pop;
           T* b = (T*)*swap;
-          const bool f = wf && k == nl - 1;
+          const bool f = (wf || wtile) && k == nl - 1;
+          // (a run of two-pass steps leaves n and psi of its last step)
           const hipError_t e =
-              k >= nl - nquad
-                  ? tile(s, a, b, f ? n : nullptr, psi, u)
-                  : fused_regs(s, a, b);
+              k >= nl - nquad ? tile(s, wtile, a, b, f ? n : nullptr, psi, wf ? u : nullptr)
+              : wtile         ? two_pass(s, a, b, n, psi, u, false)
+                              : fused_regs(s, a, b);
           if (e != hipSuccess) return hip_fail(e, "idmx_sc_run launch");
           std::swap(*pop, *swap);
         }

@@ -1418,13 +1418,16 @@ __device__ inline void site_xyz(const Geom& geo, int64_t g, int& x, int& y, int&
 
 // The per-site wall masks of the fused step with walls (kWallSelf), from the
 // flags: recomputed at every run, so flags changed between runs are seen.
+// Writes 1 to *other (unless null) when a flag is neither 0 nor 1.
 template <class S>
 __global__ void __launch_bounds__(256)
-k_wall_mask(const uint8_t* __restrict__ walls, Geom geo, uint64_t* __restrict__ mask) {
+k_wall_mask(const uint8_t* __restrict__ walls, Geom geo, uint64_t* __restrict__ mask,
+            uint32_t* __restrict__ other) {
   for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < geo.V;
        g += (int64_t)gridDim.x * blockDim.x) {
     int x, y, z;
     site_xyz(geo, g, x, y, z);
+    if (other && walls[g] > 1) *other = 1;
     uint64_t m = walls[g] != 1 ? (uint64_t(1) << kWallSelf) : uint64_t(0);
 #pragma unroll
     for (int q = 1; q < S::Q; q++) {

@@ -32,11 +32,15 @@ struct TileShape {
   static constexpr int F0 = CW(0) * CW(0), F1 = KS > 2 ? CW(1) * CW(1) : 1;
 };
 
-template <class T, bool SHIFT, int COLL, int B, int KS, bool WF>
+// WALLS: flags 0 and 1 only; the masks and the solid sites' psi (psi_out,
+// which keeps them) are read once and kept in LDS, and a site next to a solid
+// one takes the population that would stream in from there from its own f*.
+// u_out may then be null.
+template <class T, bool SHIFT, int COLL, int B, int KS, bool WF, bool WALLS = false>
 __global__ void __launch_bounds__((TileShape<B, KS>::NT))
 k_tile2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> P, int ntx,
-         int ntiles, double* __restrict__ n_out, double* __restrict__ psi_out,
-         double* __restrict__ u_out) {
+         int ntiles, double* __restrict__ n_out, double* psi_out, double* __restrict__ u_out,
+         const uint64_t* __restrict__ wmask = nullptr, T bx = T(0), T by = T(0)) {
   using S = D2Q9;
   using ES = D2E4;
   using SH = TileShape<B, KS>;
@@ -45,6 +49,10 @@ k_tile2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
   __shared__ T fa[Q][SH::F0], fb[Q][SH::F1];
   __shared__ T pa[SH::PW(0) * SH::PW(0)], pb[SH::PW(1) * SH::PW(1)];
   __shared__ T tab[NTAB];
+  // masks and psi of the solid sites of stage 0's region
+  constexpr int W0 = WALLS ? SH::PW(0) : 1;
+  __shared__ T pwall[W0 * W0];
+  __shared__ uint32_t wall[W0 * W0];
   const int per = gridDim.x >> 3;
   const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if (tile >= ntiles) return;
@@ -62,6 +70,9 @@ k_tile2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
     constexpr int IW = s > 0 ? SH::CW(s - 1) : 1;  // width of the region fin covers
     const bool in = tid < PW * PW;
     const int px = tid % PW, py = tid / PW;
+    // this site in stage 0's region
+    const int w0 = WALLS ? (py + (W0 - PW) / 2) * W0 + px + (W0 - PW) / 2 : 0;
+    uint32_t m = 0;
     T f[Q], dn = T(0);
     if (in) {
       if constexpr (s == 0) {
@@ -71,38 +82,59 @@ k_tile2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
         const int64_t g = (int64_t)y * geo.L0 + x;
 #pragma unroll
         for (int q = 0; q < Q; q++) f[q] = pop_ld(pop, q, geo.V, g);
+        if constexpr (WALLS) {
+          m = (uint32_t)wmask[g];
+          wall[w0] = m;
+          pwall[w0] = (T)psi_out[g];
+        }
       } else {
+        if constexpr (WALLS) m = wall[w0];
         // f streamed from the previous stage's f*: its region reaches one
         // site further on every side
 #pragma unroll
         for (int q = 0; q < Q; q++)
-          f[q] = fin[q * fin_n + (py + 1 - S::cy[q]) * IW + px + 1 - S::cx[q]];
+          f[q] = WALLS && q > 0 && (m >> opposite<S>(q) & 1)
+                     ? fin[opposite<S>(q) * fin_n + (py + 1) * IW + px + 1]
+                     : fin[q * fin_n + (py + 1 - S::cy[q]) * IW + px + 1 - S::cx[q]];
       }
       dn = f[0];
 #pragma unroll
       for (int q = 1; q < Q; q++) dn += f[q];
-      psi[tid] = psi_of(P.psi_kind, SHIFT ? P.rho0 + dn : dn);
+      psi[tid] = WALLS && (m >> kWallSelf & 1) ? pwall[w0]
+                                               : psi_of(P.psi_kind, SHIFT ? P.rho0 + dn : dn);
     }
     __syncthreads();
     if (in && px > 0 && px < PW - 1 && py > 0 && py < PW - 1) {
       T gx, gy, gz, fo[Q], u[3];
       iso_grad<ES>([&](int e) { return psi[tid + ES::ey[e] * PW + ES::ex[e]]; }, gx, gy, gz);
       const T lpsi = psi[tid];
-      collide<S, T, SHIFT, COLL>(f, dn, gx, gy, T(0), lpsi, PL, fo, u);
+      collide<S, T, SHIFT, COLL, WALLS>(f, dn, gx, gy, T(0), lpsi, PL, fo, u, bx, by);
       if constexpr (s < KS - 1) {
         const int c = (py - 1) * CW + px - 1;
 #pragma unroll
         for (int q = 0; q < Q; q++) fout[q * fout_n + c] = fo[q];
       } else {
         const int x = x0 + px - 1, y = y0 + py - 1;
-        if (x < geo.L0 && y < geo.L1) {
-          push_store<S, T>(pop_swap, geo, x, y, 0, fo);
+        if (x < geo.L0 && y < geo.L1 && !(WALLS && (m >> kWallSelf & 1))) {
+          const int64_t g = (int64_t)x + (int64_t)geo.L0 * y;
+          if (WALLS && m != 0) {
+            // aimed at a solid site: back to this one as the opposite
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+              const int xt = wrap(x + S::cx[q], geo.L0), yt = wrap(y + S::cy[q], geo.L1);
+              if (q > 0 && (m >> q & 1)) pop_st_nt(pop_swap, opposite<S>(q), geo.V, g, fo[q]);
+              else pop_st_nt(pop_swap, q, geo.V, lex(geo, xt, yt, 0), fo[q]);
+            }
+          } else {
+            push_store<S, T>(pop_swap, geo, x, y, 0, fo);
+          }
           if (WF) {
-            const int64_t g = (int64_t)x + (int64_t)geo.L0 * y;
             n_out[g] = (double)(SHIFT ? P.rho0 + dn : dn);
             psi_out[g] = (double)lpsi;
-            u_out[g] = (double)u[0];
-            u_out[g + geo.V] = (double)u[1];
+            if (!WALLS || u_out) {
+              u_out[g] = (double)u[0];
+              u_out[g + geo.V] = (double)u[1];
+            }
           }
         }
       }

@@ -80,9 +80,11 @@ enum {
                                 reference's own structure */
   IDMX_RUN_FUSED_WALLS = 4   /* with walls (FP64 BGK, E4): the fused step with
                                 walls on any lattice size (by default it is
-                                used from 2^19 sites up, the two-pass step
-                                below; the last step of a run that writes the
-                                fields is always the two-pass one) */
+                                used from 2^19 sites up, and below on 2D
+                                lattices several steps per launch, where the
+                                run has at least 8, or the two-pass step; a
+                                single last step of a run that writes the
+                                fields is the two-pass one) */
 };
 
 typedef struct idmx_ctx_s* idmx_ctx_t;

@@ -115,3 +115,49 @@ def test_small_3d_step_equals_march(tenet, es, dims, prec, coll, wf):
         else:
             # ~10 roundings of 6e-8 of the largest value per step
             assert np.abs(r - g).max() <= 5 * 10 * 6e-8 * np.abs(r).max()
+
+
+@pytest.mark.parametrize('dims,g,other', [((5, 7), 0.0, False), ((40, 9), 1e-5, False),
+                                          ((123, 130), 2e-5, False), ((250, 131), 0.0, False),
+                                          ((61, 50), 1e-5, True), ((700, 640), 1e-5, False),
+                                          ((700, 640), 0.0, True)])
+@pytest.mark.parametrize('steps,wf', [(7, True), (8, False), (11, True), (17, False)])
+def test_small_2d_walls_equal_two_pass(tenet, dims, g, other, steps, wf):
+    """Walls on the tiles: solid sites across the periodic edges and between
+    tiles; with a flag that is neither 0 nor 1 the run stays on the two-pass
+    step. Same arithmetic in the same order on the fluid sites."""
+    from idmx.IdpyCode import IdpyMemory
+    from idmx.LBM._base import PopArray
+    from idmx.LBM._engine import SCEngine
+    rng = np.random.default_rng(6)
+    V = int(np.prod(dims))
+    w = np.where(rng.random(V) < 0.2, 0, 1).astype(np.uint8)
+    w[:dims[0]] = 0
+    if other:
+        w[V // 2:V // 2 + 3] = 2
+    psi_w = np.where(w != 1, rng.uniform(0.3, 0.7, size=V), 0.0)
+    n0 = 1.0 + 0.3 * np.sin(2 * np.pi * np.arange(V) / 17 + 0.3)
+    fl = w == 1
+    wd = IdpyMemory.OnDevice(w, tenet)
+    out = []
+    for two_pass in (True, False):
+        eng = SCEngine(tenet, 'D2Q9', 'D2E4', dims, 'exp', -5.0 / 3.0, 1.0)
+        eng.set_walls(wd)
+        if g:
+            eng.set_body_force(0.0, g, 0.0)
+        n = IdpyMemory.OnDevice(n0, tenet)
+        psi = IdpyMemory.OnDevice(psi_w, tenet)
+        u = IdpyMemory.Zeros(2 * V, np.float64, tenet)
+        a, b = PopArray(eng, tenet), PopArray(eng, tenet)
+        eng.init_pop(a, n, u)
+        eng.init_pop(b, n, u)
+        swapped = eng.run(a, b, steps, n=n, psi=psi, u=u, write_fields=wf, two_pass=two_pass)
+        assert swapped == (steps % 2 == 1)
+        out.append((eng.pop_to_host_soa(b if swapped else a).reshape(9, V)[:, fl], n.D2H()[fl],
+                    psi.D2H(), u.D2H().reshape(2, V)[:, fl]))
+        for x in (n, psi, u, a, b):
+            x.Free()
+        eng.close()
+    wd.Free()
+    for r, t in zip(*out):
+        assert np.isfinite(t).all() and np.array_equal(r, t)
