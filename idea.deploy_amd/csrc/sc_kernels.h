@@ -305,25 +305,27 @@ __device__ inline void collide(const T (&f)[S::Q], T dn, T gx, T gy, T gz,
     // idpy/LBM/MultiPhaseKernels.py:132-216): the equilibrium velocity is
     // u + F/(n omega), no Guo term, and the velocity written is the mean of
     // the pre- and post-collision velocities.
-    const T om = P.omega;
-    const T u0x = jx / n, u0y = jy / n, u0z = S::D == 3 ? jz / n : T(0);
-    const T lux = u0x + Fx / n / om, luy = u0y + Fy / n / om;
-    const T luz = S::D == 3 ? u0z + Fz / n / om : T(0);
-    const T uu = lux * lux + luy * luy + luz * luz;
-    const T eu = T(-0.5) * uu * T(kCM2);
-    auto relax = [&](int q, T e) {
-      T feq = e * n * T(S::w[q]);
-      if (SHIFT) feq -= T(S::w[q]) * P.rho0;
-      fo[q] = f[q] * (T(1) - om) + feq * om;
-    };
-    relax(0, T(1) + eu);
+    // Evaluated pair by pair as below: with a = omega n,
+    //   f* = (1 - om) f + w [om n - (3/2) a u.u + (9/2) a (xi.u)^2] + 3 w a xi.u
+    const T om = P.omega, c_f = T(1) - om;
+    const T inv_n = T(1) / n, sF = inv_n * (T(1) / om);
+    const T u0x = jx * inv_n, u0y = jy * inv_n, u0z = S::D == 3 ? jz * inv_n : T(0);
+    const T lux = u0x + Fx * sF, luy = u0y + Fy * sF;
+    const T luz = S::D == 3 ? u0z + Fz * sF : T(0);
+    const T a = om * n, ax = a * lux, ay = a * luy, az = a * luz;
+    T au = ax * lux + ay * luy;
+    if (S::D == 3) au += az * luz;
+    // (n - rho0 rather than dn: the two-pass step has only n)
+    const T A = om * (SHIFT ? n - P.rho0 : n) - T(0.5 * kCM2) * au;
+    fo[0] = c_f * f[0] + T(S::w[0]) * A;
 #pragma unroll
     for (int p = 0; p < S::NPAIR; p++) {
       const int q = S::PairQ[p], o = S::opp[q];
-      const T xu = xi_dot<S>(q, lux, luy, luz);
-      const T e1 = xu * T(kCM2), e2 = T(0.5) * xu * xu * T(kCM4);
-      relax(q, T(1) + (e1 + e2) + eu);
-      relax(o, T(1) + (e2 - e1) + eu);
+      const T xa = xi_dot<S>(q, ax, ay, az);
+      const T ev = T(S::w[q] * 0.5 * kCM4) * (xa * xi_dot<S>(q, lux, luy, luz)) + T(S::w[q]) * A;
+      const T od = T(S::w[q] * kCM2) * xa;
+      fo[q] = c_f * f[q] + (ev + od);
+      fo[o] = c_f * f[o] + (ev - od);
     }
     T px = 0, py = 0, pz = 0;
 #pragma unroll
@@ -335,9 +337,9 @@ __device__ inline void collide(const T (&f)[S::Q], T dn, T gx, T gy, T gz,
       if (S::cz[q] == 1) pz += fo[q];
       if (S::cz[q] == -1) pz -= fo[q];
     }
-    u[0] = T(0.5) * (u0x + px / n);
-    u[1] = T(0.5) * (u0y + py / n);
-    u[2] = S::D == 3 ? T(0.5) * (u0z + pz / n) : T(0);
+    u[0] = T(0.5) * (u0x + px * inv_n);
+    u[1] = T(0.5) * (u0y + py * inv_n);
+    u[2] = S::D == 3 ? T(0.5) * (u0z + pz * inv_n) : T(0);
     return;
   }
   const T inv_n = T(1) / n;
@@ -347,33 +349,32 @@ __device__ inline void collide(const T (&f)[S::Q], T dn, T gx, T gy, T gz,
   u[0] = ux;
   u[1] = uy;
   u[2] = uz;
-  const T uu = ux * ux + uy * uy + uz * uz;
-  const T Fu = Fx * ux + Fy * uy + Fz * uz;
   if (COLL == 0 || COLL == 4) {
+    // f* = (1 - om) f + om f_eq + (1 - om/2) w [3 (xi - u).F + 9 xi.u xi.F]
+    // with f_eq = w n [1 + 3 xi.u + (9/2) (xi.u)^2 - (3/2) u.u]. Since
+    // n u = j + F/2, the terms odd in xi add up to 3 w xi.P with
+    // P = om j + F, the quadratic ones to 9 w xi.u xi.H with
+    // H = (om/2) j + (1 - om/4) F, and the rest to w A, A = om n - 3 u.H:
+    // opposite velocities share all of it (D2Q9: 90 operations instead of
+    // 170 with the terms one by one). SHIFT subtracts w rho0 from f_eq, i.e.
+    // uses dn in place of n in A.
     const T om = P.omega;
-    const T c_f = T(1) - om;
-    const T c_g = T(1) - T(0.5) * om;
-    // n-part of f_eq without the shift: SHIFT subtracts w*rho0 from f_eq,
-    // i.e. uses dn in place of n for the constant term.
-    const T n0 = SHIFT ? dn : n;
-    // opposite velocities share xi.u, xi.F and their products: those of -xi
-    // are the same numbers with the odd terms negated
-    const T cu = T(0.5 * kCM2) * uu, cF = T(kCM2) * Fu;
-    auto relax = [&](int q, T se, T sg) {
-      const T w = T(S::w[q]);
-      const T feq = w * (n0 + n * (se - cu));
-      const T fg = w * (sg - cF);
-      fo[q] = c_f * f[q] + om * feq + c_g * fg;
-    };
-    relax(0, T(0), T(0));
+    const T c_f = T(1) - om, hj = T(0.5) * om, hF = T(1) - T(0.25) * om;
+    const T Px = om * jx + Fx, Py = om * jy + Fy, Pz = S::D == 3 ? om * jz + Fz : T(0);
+    const T Hx = hj * jx + hF * Fx, Hy = hj * jy + hF * Fy;
+    const T Hz = S::D == 3 ? hj * jz + hF * Fz : T(0);
+    T uH = ux * Hx + uy * Hy;
+    if (S::D == 3) uH += uz * Hz;
+    const T A = om * (SHIFT ? dn : n) - T(kCM2) * uH;
+    fo[0] = c_f * f[0] + T(S::w[0]) * A;
 #pragma unroll
     for (int p = 0; p < S::NPAIR; p++) {
       const int q = S::PairQ[p], o = S::opp[q];
-      const T xu = xi_dot<S>(q, ux, uy, uz), xF = xi_dot<S>(q, Fx, Fy, Fz);
-      const T e1 = T(kCM2) * xu, e2 = T(0.5 * kCM4) * xu * xu;
-      const T g1 = T(kCM2) * xF, g2 = T(kCM4) * xF * xu;
-      relax(q, e1 + e2, g1 + g2);
-      relax(o, e2 - e1, g2 - g1);
+      const T ev = T(S::w[q] * kCM4) * (xi_dot<S>(q, ux, uy, uz) * xi_dot<S>(q, Hx, Hy, Hz)) +
+                   T(S::w[q]) * A;
+      const T od = T(S::w[q] * kCM2) * xi_dot<S>(q, Px, Py, Pz);
+      fo[q] = c_f * f[q] + (ev + od);
+      fo[o] = c_f * f[o] + (ev - od);
     }
     // COLL 4: BGK with Guo forcing, then the isotropy filter (D2Q9, FP64)
     if constexpr (COLL == 4) iso_filter<S, T>(fo);
@@ -425,6 +426,7 @@ __device__ inline void collide(const T (&f)[S::Q], T dn, T gx, T gy, T gz,
     }
     // Mp F from the coordinates d of the raw Guo term on w o {1, xi, xi xi}
     constexpr int NB = NBasis<S::D>::value;
+    const T uu = ux * ux + uy * uy + uz * uz, Fu = Fx * ux + Fy * uy + Fz * uz;
     T cb[NB], d[NB];
     basis_coords<S, T, SHIFT>(dn, n, ux, uy, uz, Fx, Fy, Fz, uu, Fu, cb, d);
     T mg[Q];
@@ -473,6 +475,7 @@ __device__ inline void collide(const T (&f)[S::Q], T dn, T gx, T gy, T gz,
     // f* = A f + sum_k c_k beta_k + sum_k d_k gamma_k, with c_k / d_k the
     // coordinates of f_eq / raw Guo term on w∘{1, xi_a, xi_a xi_b}.
     constexpr int NB = NBasis<S::D>::value;
+    const T uu = ux * ux + uy * uy + uz * uz, Fu = Fx * ux + Fy * uy + Fz * uz;
     T c[NB], d[NB];
     basis_coords<S, T, SHIFT>(dn, n, ux, uy, uz, Fx, Fy, Fz, uu, Fu, c, d);
 #pragma unroll
