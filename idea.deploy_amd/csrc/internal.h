@@ -34,19 +34,28 @@ struct idmx_ctx_s {
 
 struct SimOps;
 
-// Sites from which a 2D run on the x-shifted storage (variant 10, the default
-// launch there; the Shan-Chen forcing and the isotropy filter) takes two steps
-// per launch.
-constexpr int64_t kPairSites = 3 << 17;
-// Steps per launch below that (E4 force).
-constexpr int kTileSteps = 4;
-
 // Sites below which a 3D simulation that was given no launch takes its steps
 // without a march (k_tile3d): 24^3 MRT 7.6 us per step against 13.1, 48 x 44 x
 // 40 11.6 against 14.1 (E8: 16.5 against 19.5), 60 x 50 x 48 BGK 19.3 against
 // 21.4, 64^3 25.9 against 23.6; in FP32 48 x 44 x 40 8.4 against 10.4, 50^3
 // 13.7 against 12.7.
 constexpr int64_t kTile3Sites = 150000, kTile3Sites32 = 100000;
+
+// March length of a 3D step of which two blocks share a CU: the launch runs in
+// rounds of 512 blocks of h + 2R planes each, and the least total wins (half a
+// plane for a block's start). `tiles` per plane, Lm planes; *cost: the total.
+inline int march_planes(int64_t tiles, int Lm, int R, double* cost = nullptr) {
+  double least = 1e300;
+  int best = Lm;
+  for (int nseg = 1; nseg <= std::min(Lm, 4096); nseg++) {
+    const int h = (Lm + nseg - 1) / nseg;
+    const int64_t rounds = (tiles * ((Lm + h - 1) / h) + 511) / 512;
+    const double c = (double)rounds * (h + 2 * R + 0.5);
+    if (c < least) least = c, best = h;
+  }
+  if (cost) *cost = least;
+  return best;
+}
 
 struct idmx_sc_s {
   idmx_ctx_s* ctx = nullptr;

@@ -397,8 +397,8 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
     s->tx = d->dims[0] >= 256 ? 256 : 64;
     s->ty = 1;
     // several steps per launch: two on large lattices (Impl::pair_plan), four
-    // on small ones with the E4 force (Impl::tile)
-    if (V >= kPairSites || R == 1) s->hist = 10;
+    // or two on small ones (Impl::tile)
+    s->hist = 10;
   } else {
     s->tx = 32;
     s->ty = 8;
@@ -413,12 +413,10 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
     H = std::max(H, blocks_at_8 >= 256 ? 8 : (D == 2 ? 1 : 2));
     s->H = std::min(H, Lm);
     // 3D lattices that fill the chip: the LDS-staged step on the x-shifted
-    // storage. Two of its blocks share a CU, so the launch runs in rounds of
-    // 512 blocks of H + 2R planes each, and the tile and H with the least
-    // total win (one full round where the lattice allows it: 150 x 101 x 93
-    // 127 us per step at 32 x 8, H = 14, 455 blocks, against 142 at H = 8;
-    // 200^3 MRT 592 us at 64 x 4, H = 40, against 816 with registers). A
-    // plane of 32 x 8 takes 6 % longer than one of 64 x 4 (shorter rows), but
+    // storage, with the tile and H of the least total (march_planes; one full
+    // round where the lattice allows it: 150 x 101 x 93 127 us per step at
+    // 32 x 8, H = 14, 455 blocks, against 142 at H = 8; 200^3 MRT 592 us at
+    // 64 x 4, H = 40, against 816 with registers). A plane of 32 x 8 takes 6 % longer than one of 64 x 4 (shorter rows), but
     // pads less on most widths. Reach-2 stencils in FP64 leave one block per
     // CU and stay on registers (96^3 E8: 86 us against 131), as does the dense
     // MRT collision, which is bound by its 741 products (128^3: 503 us against
@@ -433,17 +431,15 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
         if ((tx == 32 && s->coll == 3) || !s->ops->launch_ok(tx, ty, 10)) continue;
         const int64_t tiles =
             (int64_t)((s->geo.L0 + tx - 1) / tx) * ((s->geo.L1 + ty - 1) / ty);
-        for (int nseg = 1; nseg <= std::min(Lm, 4096); nseg++) {
-          const int h = (Lm + nseg - 1) / nseg;
-          const int64_t rounds = (tiles * ((Lm + h - 1) / h) + 511) / 512;
-          const double c = (double)rounds * (h + 2 * R + 0.5) * (tx == 32 ? 1.06 : 1.0);
-          if (c < least) {
-            least = c;
-            s->tx = tx;
-            s->ty = ty;
-            s->H = h;
-            s->hist = 10;
-          }
+        double c;
+        const int h = march_planes(tiles, Lm, R, &c);
+        if (tx == 32) c *= 1.06;
+        if (c < least) {
+          least = c;
+          s->tx = tx;
+          s->ty = ty;
+          s->H = h;
+          s->hist = 10;
         }
       }
     }

@@ -104,7 +104,12 @@ struct Impl {
       const int ntx = (g.L0 + TX - 1) / TX;
       const int nty = S::D == 3 ? (g.L1 + TY - 1) / TY : 1;
       const int Lm = S::D == 3 ? g.L2 : g.L1;
-      const int H = std::min(s->H, Lm);
+      // 3D: a march for these tiles, not for the tile that the step without
+      // walls runs (77 x 68 x 278: 163 us per step, 220 with the H of 32 x 8;
+      // 96^3 86 and 111)
+      const int H = S::D == 3 && s->auto_launch
+                        ? march_planes((int64_t)ntx * nty, Lm, ES::R)
+                        : std::min(s->H, Lm);
       const int nseg = (Lm + H - 1) / H;
       const int ntiles = ntx * nty * nseg;
       const unsigned grid = (unsigned)((ntiles + 7) / 8 * 8);
@@ -237,11 +242,13 @@ struct Impl {
     }
     return least;
   }
-  // Below 3 * 2^17 sites the march is a chain of too few blocks: 512^2 10.8 us
-  // per step against 10.8 with single steps, 256^2 9.5 against 6.4 (1024^2
-  // MRT: 21.8 against 38.6). A lattice much narrower than a block leaves its
-  // lanes idle.
-  // With walls (1024 x 768: 20.3 us per step, single steps 34.6) 128 threads
+  // Below 2^19 sites (reach 2 in FP64: 3 * 2^17) tiles are faster (k_tile2d:
+  // 800 x 640 BGK 10.9 us per step against 13.3, MRT 13.9 and 15.1, FP32 8.7
+  // and 10.4, E8 17.3 and 16.3; 1000 x 613 BGK 14.6 and 13.6, E8 20.6 and
+  // 17.4). A lattice much narrower than a block leaves its lanes idle.
+  static constexpr int64_t kPairSites =
+      ES::R == 2 && sizeof(T) == 8 ? 3 << 17 : int64_t(1) << 19;
+  // With walls (1024 x 768: 18.3 us per step, single steps 34.6) 128 threads
   // where both cost the same (256: 23.6, its waves longer in each other's
   // barrier; 700 x 900 18.9 and 20.0).
   static PairPlan pair_plan(const idmx_sc_s* s, bool walls) {
@@ -299,39 +306,62 @@ struct Impl {
     }
   }
 
-  // Four steps in one launch on a small 2D lattice (k_tile2d).
-  static constexpr bool kTile = S::D == 2 && ES::R == 1;
-  template <int B, bool WF, bool WALLS = false>
+  // Several steps in one launch on a small 2D lattice (k_tile2d): KS steps of
+  // B x B tiles.
+  static constexpr bool kTile = S::D == 2;
+  struct TilePlan {
+    int B = 0, KS = 0;
+  };
+  // Four steps per launch where the launch and the round trip weigh most (E4:
+  // FP64 below 10^5 sites, FP32 below 2 10^5), two where the redundant
+  // collisions do (512^2 FP64 BGK 6.3 us per step, with four 8.6). 8 x 8 tiles
+  // while every one has a CU of its own (128^2: 1.73 against 2.14), then 16 x
+  // 16. With two steps 24 x 24 from 10^5 sites (512^2 6.3 against 7.8), not
+  // with MRT, whose collisions hold more registers (7.6 against 8.5). Reach 2:
+  // two steps, 16 x 16 (256^2 E8 3.3; 22 x 22 3.9), in FP32 BGK 22 x 22 from
+  // 2 10^5 sites (512^2 5.4 against 6.5).
+  static TilePlan tile_plan(const Geom& g) {
+    constexpr bool f32 = sizeof(T) == 4, mrt = COLL == 1 || COLL == 2;
+    const bool b8 = (int64_t)((g.L0 + 7) / 8) * ((g.L1 + 7) / 8) <= 256;
+    if (ES::R == 1 && g.V < (f32 ? 200000 : 100000)) return {b8 ? 8 : 16, 4};
+    if (!mrt && g.V >= (ES::R == 1 ? 100000 : 200000) && (ES::R == 1 || f32))
+      return {kTileWide, 2};
+    return {b8 ? 8 : 16, 2};
+  }
+  static constexpr int kTileWide = ES::R == 1 ? 24 : 22;
+  template <int B, int KS, bool WF, bool WALLS = false>
   static hipError_t launch_tile(idmx_sc_s* s, const T* pop, T* swap, double* n, double* psi,
                                 double* u) {
     const Geom& g = s->geo;
     const int ntx = (g.L0 + B - 1) / B, ntiles = ntx * ((g.L1 + B - 1) / B);
     const unsigned grid = (unsigned)((ntiles + 7) / 8 * 8);
-    hipLaunchKernelGGL((k_tile2d<T, SHIFT, COLL, B, kTileSteps, WF, WALLS>), dim3(grid),
-                       dim3(TileShape<B, kTileSteps>::NT), 0, s->ctx->stream, pop, swap, g,
+    hipLaunchKernelGGL((k_tile2d<ES, T, SHIFT, COLL, B, KS, WF, WALLS>), dim3(grid),
+                       dim3(TileShape<B, KS, ES::R>::NT), 0, s->ctx->stream, pop, swap, g,
                        phys(s), ntx, ntiles, n, psi, u, (const uint64_t*)s->wmask_dev,
                        (T)s->bforce[0], (T)s->bforce[1]);
     return hipGetLastError();
   }
-  static hipError_t tile(idmx_sc_s* s, bool walls, const T* pop, T* swap, double* n, double* psi,
-                         double* u) {
+  template <int B, int KS>
+  static hipError_t launch_tile(idmx_sc_s* s, bool walls, const T* pop, T* swap, double* n,
+                                double* psi, double* u) {
+    if constexpr (kFusedWalls)
+      if (walls)
+        return n ? launch_tile<B, KS, true, true>(s, pop, swap, n, psi, u)
+                 : launch_tile<B, KS, false, true>(s, pop, swap, n, psi, u);
+    return n ? launch_tile<B, KS, true>(s, pop, swap, n, psi, u)
+             : launch_tile<B, KS, false>(s, pop, swap, n, psi, u);
+  }
+  static hipError_t tile(idmx_sc_s* s, const TilePlan& p, bool walls, const T* pop, T* swap,
+                         double* n, double* psi, double* u) {
     if constexpr (kTile) {
-      // 8 x 8 tiles while every one has a CU of its own (128^2: 1.92 us per
-      // step against 2.50), else 16 x 16 (256^2: 2.53 against 4.24)
-      const bool b8 = (int64_t)((s->geo.L0 + 7) / 8) * ((s->geo.L1 + 7) / 8) <= 256;
-      if constexpr (kFusedWalls)
-        if (walls) {
-          if (b8)
-            return n ? launch_tile<8, true, true>(s, pop, swap, n, psi, u)
-                     : launch_tile<8, false, true>(s, pop, swap, n, psi, u);
-          return n ? launch_tile<16, true, true>(s, pop, swap, n, psi, u)
-                   : launch_tile<16, false, true>(s, pop, swap, n, psi, u);
-        }
-      if (b8)
-        return n ? launch_tile<8, true>(s, pop, swap, n, psi, u)
-                 : launch_tile<8, false>(s, pop, swap, n, psi, u);
-      return n ? launch_tile<16, true>(s, pop, swap, n, psi, u)
-               : launch_tile<16, false>(s, pop, swap, n, psi, u);
+      if constexpr (ES::R == 1)
+        if (p.KS == 4)
+          return p.B == 8 ? launch_tile<8, 4>(s, walls, pop, swap, n, psi, u)
+                          : launch_tile<16, 4>(s, walls, pop, swap, n, psi, u);
+      if constexpr (COLL != 1 && COLL != 2 && (ES::R == 1 || sizeof(T) == 4))
+        if (p.B == kTileWide) return launch_tile<kTileWide, 2>(s, walls, pop, swap, n, psi, u);
+      return p.B == 8 ? launch_tile<8, 2>(s, walls, pop, swap, n, psi, u)
+                      : launch_tile<16, 2>(s, walls, pop, swap, n, psi, u);
     } else {
       return hipErrorInvalidConfiguration;
     }
@@ -421,10 +451,10 @@ struct Impl {
     // sites up, or when asked for: on smaller lattices two passes are as
     // fast as single fused steps; measured 0.94x at 64^3, 1.07x at 1024^2,
     // 1.30x at 256^3 and 1.47x at 4096^2)
-    bool fwalls = kFusedWalls && s->walls && (flags & IDMX_RUN_TWO_PASS) == 0 &&
+    const bool fwalls = kFusedWalls && s->walls && (flags & IDMX_RUN_TWO_PASS) == 0 &&
                         s->desc.psi_kind != IDMX_PSI_PROGRAM &&
                         (s->geo.V >= (int64_t(1) << 19) || (flags & IDMX_RUN_FUSED_WALLS) != 0);
-    bool twop = !fwalls && ((flags & IDMX_RUN_TWO_PASS) != 0 || s->walls || body ||
+    const bool twop = !fwalls && ((flags & IDMX_RUN_TWO_PASS) != 0 || s->walls || body ||
                                   s->desc.psi_kind == IDMX_PSI_PROGRAM);
     if ((twop || fwalls) && (!n || !psi)) {
       set_error(s->walls || body || s->desc.psi_kind == IDMX_PSI_PROGRAM
@@ -463,25 +493,20 @@ struct Impl {
     }
     // smaller 2D lattices with walls: several steps per launch, if every flag
     // is 0 or 1 (waiting for that costs 10 us; a run of 8 steps of 128^2
-    // takes 45 us then, 69 on two passes). Two on the pair kernel where that
-    // applies (700 x 640 14.1 us per step; tiles 18.5, two passes 23.1), else
-    // kTileSteps on tiles (128^2 2.2 against 6.9, 256^2 2.9 against 8.0, 512^2
-    // 10.8 against 14.8, 150 x 2000 13.3 against 16.8). A run of two-pass
-    // steps leaves n and psi of its last step: so do the tiles, while the
-    // pairs are left to runs that ask for them.
+    // takes 45 us then, 69 on two passes): tiles as without walls (128^2 1.9
+    // us per step, two passes 6.9; 256^2 2.6 and 8.0, 512^2 6.7 and 14.8, 800
+    // x 640 11.6 and 25). A run of two-pass steps leaves n and psi of its last
+    // step, and so does this one.
     bool wtile = false;
     if constexpr (kTile && kFusedWalls)
       if (twop && s->walls && (flags & IDMX_RUN_TWO_PASS) == 0 && !pev &&
-          s->desc.psi_kind != IDMX_PSI_PROGRAM && s->wmask_dev && nsteps >= 2 * kTileSteps) {
+          s->desc.psi_kind != IDMX_PSI_PROGRAM && s->wmask_dev && nsteps >= 8) {
         *s->wflag_host = 0;
         hipLaunchKernelGGL((k_wall_mask<S>), dim3(grid_for(s->geo.V)), dim3(256), 0, st, s->walls,
                            s->geo, s->wmask_dev, s->wflag_host);
         IDMX_HIP(hipGetLastError());
         IDMX_HIP(hipStreamSynchronize(st));
-        if (*s->wflag_host == 0) {
-          if (wf && pair_plan(s, true).nt) fwalls = true, twop = false;
-          else wtile = true;
-        }
+        wtile = *s->wflag_host == 0;
       }
     IDMX_HIP(hipEventRecord(s->ctx->ev0, st));
     // pull-form variants: convert the streamed populations to the pull form,
@@ -494,8 +519,8 @@ struct Impl {
     // steps reads the streamed storage, the last writes it (the step that
     // writes n/psi/u runs on the streamed storage), so a run of one step
     // never leaves it
-    // (small 2D lattices with the E4 force stay on the streamed storage on
-    // variant 10: kTileSteps steps per launch, single steps with registers)
+    // (small 2D lattices stay on the streamed storage on variant 10: several
+    // steps per launch on tiles, single steps with registers)
     const bool small = kTile && !fwalls && s->geo.V < kPairSites;
     // small 3D lattices, unless a launch was set: k_tile3d
     const bool small3 = S::D == 3 && !twop && !fwalls && s->auto_launch &&
@@ -530,22 +555,23 @@ struct Impl {
         std::swap(*pop, *swap);
       }
     }
-    // kTileSteps steps per launch, an even number of such launches for the same
+    // tp.KS steps per launch, an even number of such launches for the same
     // reason; they and the single steps before them keep the streamed storage
     int nquad = 0;
+    const TilePlan tp = kTile ? tile_plan(s->geo) : TilePlan{};
     if constexpr (kTile)
       if (wtile || (small && !twop && !pev && (COLL >= 3 || s->hist == 10)))
-        nquad = nsteps / kTileSteps & ~1;
+        nquad = nsteps / tp.KS & ~1;
     if constexpr (kTile)
       if (nquad > 0) {
-        const int nl = nsteps - nquad * (kTileSteps - 1);
+        const int nl = nsteps - nquad * (tp.KS - 1);
         for (int k = 0; k < nl; k++) {
           const T* a = (const T*)*pop;
           T* b = (T*)*swap;
           const bool f = (wf || wtile) && k == nl - 1;
           // (a run of two-pass steps leaves n and psi of its last step)
           const hipError_t e =
-              k >= nl - nquad ? tile(s, wtile, a, b, f ? n : nullptr, psi, wf ? u : nullptr)
+              k >= nl - nquad ? tile(s, tp, wtile, a, b, f ? n : nullptr, psi, wf ? u : nullptr)
               : wtile         ? two_pass(s, a, b, n, psi, u, false)
                               : fused_regs(s, a, b);
           if (e != hipSuccess) return hip_fail(e, "idmx_sc_run launch");

@@ -1,21 +1,23 @@
-// sc_tile.h -- steps of small lattices: four time steps of a D2Q9 lattice (E4
-// force) in one launch (k_tile2d), one step of a D3Q19 lattice without a
+// sc_tile.h -- steps of small lattices: two or four time steps of a D2Q9
+// lattice in one launch (k_tile2d), one step of a D3Q19 lattice without a
 // march (k_tile3d).
 //
 // What bounds a small lattice is latency: a step of 128^2 sites moves 2.4 MB
 // that stay in L2 and is over in 5.2 us, most of it launch, two memory
 // latencies and a barrier. A block here loads a B x B tile with the ring of
 // sites that KS steps reach, takes the steps in LDS on a region that shrinks
-// by two sites per side and step, and pushes the result: one launch and one
-// round trip to memory per KS steps, paid for with redundant collisions on
-// the ring (KS = 4: 3.4 times the sites of an 8 x 8 tile, 2.0 of a 16 x 16
-// one), which an otherwise idle chip has room for. Measured per step against
-// the register step, one launch each: 128^2 1.92 us (5.10), 256^2 2.53 (6.06),
-// 384^2 6.6 (8.6), 512^2 9.5 (11.0).
+// by R + 1 sites per side and step (R the reach of the force stencil), and
+// pushes the result: one launch and one round trip to memory per KS steps,
+// paid for with redundant collisions on the ring (E4, KS = 4: 3.4 times the
+// sites of an 8 x 8 tile, 2.0 of a 16 x 16 one; KS = 2: 1.2 of a 24 x 24 one),
+// which an otherwise idle chip has room for; from about 10^5 sites the FP64
+// vector units bound it. Measured per step against the register step, one
+// launch each: E4 128^2 1.73 us (5.10), 256^2 2.3 (6.06), 512^2 6.3 (11.0);
+// E8 128^2 2.5 (7.0), 256^2 3.3 (8.2), 620^2 13.7 (26.5), in FP32 7.4 (16.2).
 //
 // One site per thread: thread t is site (t mod w, t / w) of the stage's
 // region of w x w sites, where psi is needed (PW); it collides there unless
-// it lies on the region's rim.
+// it lies within R of the region's rim.
 #pragma once
 #include <type_traits>
 
@@ -23,10 +25,11 @@
 
 namespace idmx {
 
-template <int B, int KS>
+template <int B, int KS, int R>
 struct TileShape {
-  static constexpr int PW(int s) { return B + 4 * (KS - 1 - s) + 2; }  // psi of stage s
-  static constexpr int CW(int s) { return PW(s) - 2; }                 // collisions
+  // psi of stage s, collisions
+  static constexpr int PW(int s) { return B + 2 * ((R + 1) * (KS - 1 - s) + R); }
+  static constexpr int CW(int s) { return PW(s) - 2 * R; }
   static constexpr int NT = (PW(0) * PW(0) + 63) / 64 * 64;
   // f* of even and odd stages (that of the last one goes to memory)
   static constexpr int F0 = CW(0) * CW(0), F1 = KS > 2 ? CW(1) * CW(1) : 1;
@@ -36,14 +39,14 @@ struct TileShape {
 // which keeps them) are read once and kept in LDS, and a site next to a solid
 // one takes the population that would stream in from there from its own f*.
 // u_out may then be null.
-template <class T, bool SHIFT, int COLL, int B, int KS, bool WF, bool WALLS = false>
-__global__ void __launch_bounds__((TileShape<B, KS>::NT))
+template <class ES, class T, bool SHIFT, int COLL, int B, int KS, bool WF, bool WALLS = false>
+__global__ void __launch_bounds__((TileShape<B, KS, ES::R>::NT))
 k_tile2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> P, int ntx,
          int ntiles, double* __restrict__ n_out, double* psi_out, double* __restrict__ u_out,
          const uint64_t* __restrict__ wmask = nullptr, T bx = T(0), T by = T(0)) {
   using S = D2Q9;
-  using ES = D2E4;
-  using SH = TileShape<B, KS>;
+  constexpr int R = ES::R;
+  using SH = TileShape<B, KS, R>;
   constexpr int Q = S::Q, NB = NBasis<2>::value;
   constexpr int NTAB = COLL == 2 ? Q : COLL == 1 ? Q * Q + 2 * NB * Q : 1;
   __shared__ T fa[Q][SH::F0], fb[Q][SH::F1];
@@ -76,7 +79,7 @@ k_tile2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
     T f[Q], dn = T(0);
     if (in) {
       if constexpr (s == 0) {
-        const int D = 2 * KS - 1;
+        constexpr int D = (R + 1) * (KS - 1) + R;
         const int x = ((x0 - D + px) % geo.L0 + geo.L0) % geo.L0;
         const int y = ((y0 - D + py) % geo.L1 + geo.L1) % geo.L1;
         const int64_t g = (int64_t)y * geo.L0 + x;
@@ -104,17 +107,17 @@ k_tile2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
                                                : psi_of(P.psi_kind, SHIFT ? P.rho0 + dn : dn);
     }
     __syncthreads();
-    if (in && px > 0 && px < PW - 1 && py > 0 && py < PW - 1) {
+    if (in && px >= R && px < PW - R && py >= R && py < PW - R) {
       T gx, gy, gz, fo[Q], u[3];
       iso_grad<ES>([&](int e) { return psi[tid + ES::ey[e] * PW + ES::ex[e]]; }, gx, gy, gz);
       const T lpsi = psi[tid];
       collide<S, T, SHIFT, COLL, WALLS>(f, dn, gx, gy, T(0), lpsi, PL, fo, u, bx, by);
       if constexpr (s < KS - 1) {
-        const int c = (py - 1) * CW + px - 1;
+        const int c = (py - R) * CW + px - R;
 #pragma unroll
         for (int q = 0; q < Q; q++) fout[q * fout_n + c] = fo[q];
       } else {
-        const int x = x0 + px - 1, y = y0 + py - 1;
+        const int x = x0 + px - R, y = y0 + py - R;
         if (x < geo.L0 && y < geo.L1 && !(WALLS && (m >> kWallSelf & 1))) {
           const int64_t g = (int64_t)x + (int64_t)geo.L0 * y;
           if (WALLS && m != 0) {
@@ -141,11 +144,13 @@ k_tile2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
     }
     if constexpr (s < KS - 1) __syncthreads();
   };
-  static_assert(KS == 4, "stages are written out");
+  static_assert(KS == 2 || KS == 4, "stages are written out");
   stage(std::integral_constant<int, 0>{}, nullptr, 0, fa[0], SH::F0, pa);
-  stage(std::integral_constant<int, 1>{}, fa[0], SH::F0, fb[0], SH::F1, pb);
-  stage(std::integral_constant<int, 2>{}, fb[0], SH::F1, fa[0], SH::F0, pa);
-  stage(std::integral_constant<int, 3>{}, fa[0], SH::F0, nullptr, 0, pb);
+  if constexpr (KS == 4) {
+    stage(std::integral_constant<int, 1>{}, fa[0], SH::F0, fb[0], SH::F1, pb);
+    stage(std::integral_constant<int, 2>{}, fb[0], SH::F1, fa[0], SH::F0, pa);
+  }
+  stage(std::integral_constant<int, KS - 1>{}, fa[0], SH::F0, nullptr, 0, pb);
 }
 
 // --------------------------------------------------------------------------

@@ -1,5 +1,5 @@
-"""Two steps per launch (k_pair2d, 2D lattices of at least 3 * 2^17 sites on
-variant 10 and with the Shan-Chen forcing or the isotropy filter) against
+"""Two steps per launch (k_pair2d, 2D lattices of at least 2^19 sites, with E6
+/ E8 in FP64 3 * 2^17, on variant 10 and with the Shan-Chen forcing or the isotropy filter) against
 single steps: variant 9, or the two-pass step for the forcing and the filter.
 Every site sees the same arithmetic, so FP64 results are equal and FP32 ones
 may differ by the contraction of a few operations per step. Sizes lie at the
@@ -17,7 +17,10 @@ CASES = [('D2E4', (500, 787), 'fp64', 'bgk'), ('D2E4', (251, 1571), 'fp64', 'mrt
          ('D2E8', (493, 801), 'fp64', 'bgk'), ('D2E6', (4099, 97), 'fp64', 'dense'),
          ('D2E4', (123, 3201), 'fp64', 'bgk'), ('D2E4', (1499, 263), 'fp64', 'sc'),
          ('D2E8', (613, 643), 'fp64', 'iso'), ('D2E4', (749, 526), 'fp32s', 'bgk'),
-         ('D2E8', (640, 615), 'fp32s', 'mrt')]
+         ('D2E8', (640, 615), 'fp32s', 'mrt'), ('D2E4', (500, 1051), 'fp64', 'bgk'),
+         ('D2E4', (251, 2091), 'fp64', 'mrt'), ('D2E4', (123, 4301), 'fp64', 'bgk'),
+         ('D2E4', (1499, 351), 'fp64', 'sc'), ('D2E4', (749, 702), 'fp32s', 'bgk'),
+         ('D2E8', (640, 821), 'fp32s', 'mrt')]
 
 
 def _run(tenet, es, dims, prec, coll, single, steps, wf):
@@ -68,7 +71,8 @@ def test_two_steps_per_launch_equal_single_steps(tenet, es, dims, prec, coll, st
             assert np.abs(r - g).max() <= steps * 10 * 6e-8 * np.abs(r).max()
 
 
-@pytest.mark.parametrize('dims,g', [((1024, 520), 1e-5), ((613, 643), 0.0), ((251, 1571), 2e-5)])
+@pytest.mark.parametrize('dims,g', [((1024, 520), 1e-5), ((613, 643), 0.0), ((251, 1571), 2e-5),
+                                    ((251, 2091), 1e-5), ((613, 857), 0.0)])
 @pytest.mark.parametrize('steps,wf', [(3, True), (4, True), (5, False), (8, True), (11, False)])
 def test_two_steps_per_launch_with_walls(tenet, dims, g, steps, wf):
     """The walls step (plates, blocks across the periodic edges, lone solid

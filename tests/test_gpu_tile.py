@@ -1,9 +1,9 @@
-"""Four steps per launch on small 2D lattices (k_tile2d: E4 force, fewer than
-3 * 2^17 sites, the default launch) against single steps with the populations
+"""Two or four steps per launch on small 2D lattices (k_tile2d, below 2^19
+sites, with E6 / E8 in FP64 3 * 2^17, the default launch) against single steps with the populations
 in registers (variant 1), or against the two-pass step for the Shan-Chen
 forcing and the isotropy filter: the same arithmetic per site, equal in FP64
 and, contraction being the same in every launch, to rounding in FP32. Lattices
-smaller than a tile and its ring, edges of the 8 x 8 and 16 x 16 tiles, and
+smaller than a tile and its ring, edges of the 8, 16, 22 and 24 wide tiles, and
 runs that leave single steps over. Likewise one step of a small 3D lattice
 without a march (k_tile3d), on lattices shorter than its 16 x 4 x 4 tile and
 its halo and ones that leave partial tiles."""
@@ -17,10 +17,18 @@ pytestmark = pytest.mark.gpu
 CASES = [((3, 3), 'fp64', 'bgk'), ((5, 70), 'fp64', 'mrt'), ((128, 128), 'fp64', 'bgk'),
          ((127, 129), 'fp64', 'bgk'), ((129, 145), 'fp64', 'dense'), ((17, 300), 'fp64', 'sc'),
          ((8, 16), 'fp64', 'iso'), ((301, 47), 'fp64', 'bgk'), ((627, 627), 'fp64', 'mrt'),
-         ((95, 64), 'fp32s', 'bgk'), ((161, 200), 'fp32s', 'mrt')]
+         ((95, 64), 'fp32s', 'bgk'), ((161, 200), 'fp32s', 'mrt'),
+         ((385, 313), 'fp64', 'bgk'), ((337, 361), 'fp64', 'sc'), ((400, 300), 'fp64', 'iso'),
+         ((500, 401), 'fp32s', 'bgk')]
+CASES = [c + ('D2E4',) for c in CASES] + [
+    ((5, 5), 'fp64', 'bgk', 'D2E8'), ((5, 70), 'fp64', 'mrt', 'D2E6'),
+    ((127, 129), 'fp64', 'bgk', 'D2E8'), ((301, 47), 'fp64', 'iso', 'D2E8'),
+    ((161, 200), 'fp64', 'dense', 'D2E6'), ((627, 627), 'fp64', 'bgk', 'D2E6'),
+    ((95, 64), 'fp32s', 'bgk', 'D2E8'), ((463, 440), 'fp32s', 'bgk', 'D2E8'),
+    ((463, 440), 'fp32s', 'mrt', 'D2E6')]
 
 
-def _run(tenet, dims, prec, coll, single, steps, wf):
+def _run(tenet, dims, prec, coll, single, steps, wf, es='D2E4'):
     from idmx.IdpyCode import IdpyMemory
     from idmx.LBM import hermite
     from idmx.LBM._base import PopArray
@@ -30,7 +38,7 @@ def _run(tenet, dims, prec, coll, single, steps, wf):
         S[3, 4] = 0.05
     kw = {'mrt': hermite.mrt_kernel_tables('D2Q9', S)} if coll in ('mrt', 'dense') else \
         {'forcing': 'sc'} if coll == 'sc' else {'iso_filter': True} if coll == 'iso' else {}
-    eng = SCEngine(tenet, 'D2Q9', 'D2E4', dims, 'exp', -5.0 / 3.0, 1.0, precision=prec,
+    eng = SCEngine(tenet, 'D2Q9', es, dims, 'exp', -5.0 / 3.0, 1.0, precision=prec,
                    rho0=1.0, **kw)
     assert eng.get_launch()[3] == 10
     if single:
@@ -54,11 +62,11 @@ def _run(tenet, dims, prec, coll, single, steps, wf):
     return swapped, out
 
 
-@pytest.mark.parametrize('dims,prec,coll', CASES)
-@pytest.mark.parametrize('steps,wf', [(7, True), (8, True), (8, False), (13, True), (18, False)])
-def test_four_steps_per_launch_equal_single_steps(tenet, dims, prec, coll, steps, wf):
-    sw1, ref = _run(tenet, dims, prec, coll, True, steps, wf)
-    sw2, got = _run(tenet, dims, prec, coll, False, steps, wf)
+@pytest.mark.parametrize('dims,prec,coll,es', CASES)
+@pytest.mark.parametrize('steps,wf', [(3, True), (7, True), (8, True), (8, False), (13, True), (18, False)])
+def test_four_steps_per_launch_equal_single_steps(tenet, dims, prec, coll, es, steps, wf):
+    sw1, ref = _run(tenet, dims, prec, coll, True, steps, wf, es)
+    sw2, got = _run(tenet, dims, prec, coll, False, steps, wf, es)
     assert sw1 == sw2      # the state ends in the buffer where single steps leave it
     for r, g in zip(ref, got):
         assert np.isfinite(g).all()
