@@ -488,23 +488,26 @@ inline bool aligned(const void* p, size_t n) { return ((uintptr_t)p & (n - 1)) =
 
 template <int CIN, int TP>
 hipError_t conv_tile_ct(idmx_ctx_s* c, const void* in, const void* wt, const float* bias,
-                        void* out, float* out_f32, const ConvShape& s, int relu, int ct) {
+                        void* out, float* out_f32, const ConvShape& s, int relu, int ct,
+                        BwdWSum t) {
   const int P = s.N * s.H * s.W, cots = (s.Cout + 15) / 16;
-  const dim3 grid((P + TP - 1) / TP, cots / ct);
-  const size_t shm = ConvTile<CIN>::lds(s.W, TP);
+  t.nx = (P + TP - 1) / TP;
+  const int gy = cots / ct, sums = t.part ? ((t.n + 63) / 64 + gy - 1) / gy : 0;
+  const dim3 grid(t.nx + sums, gy);
+  const size_t shm = std::max<size_t>(ConvTile<CIN>::lds(s.W, TP), 256 * sizeof(float));
   auto go = [&](auto k) {
     hipLaunchKernelGGL(k, grid, dim3(256), shm, c->stream, (const uint16_t*)in,
-                       (const uint16_t*)wt, bias, (uint16_t*)out, out_f32, s, relu);
+                       (const uint16_t*)wt, bias, (uint16_t*)out, out_f32, s, relu, t);
     return hipGetLastError();
   };
   constexpr int M = ConvTile<CIN>::CTMAX;
-  if constexpr (M >= 4) {
-    if (ct == 4) return go(k_conv3x3_tile<CIN, 4, TP>);
-  }
-  if constexpr (M >= 2) {
-    if (ct == 2) return go(k_conv3x3_tile<CIN, 2, TP>);
-  }
-  return go(k_conv3x3_tile<CIN, 1, TP>);
+  if constexpr (M >= 4)
+    if (ct == 4) return t.part ? go(k_conv3x3_tile<CIN, 4, TP, true>)
+                               : go(k_conv3x3_tile<CIN, 4, TP, false>);
+  if constexpr (M >= 2)
+    if (ct == 2) return t.part ? go(k_conv3x3_tile<CIN, 2, TP, true>)
+                               : go(k_conv3x3_tile<CIN, 2, TP, false>);
+  return t.part ? go(k_conv3x3_tile<CIN, 1, TP, true>) : go(k_conv3x3_tile<CIN, 1, TP, false>);
 }
 
 // The tiled convolution where it applies (its channel counts, aligned tensors,
@@ -513,7 +516,7 @@ hipError_t conv_tile_ct(idmx_ctx_s* c, const void* in, const void* wt, const flo
 // blocks. Other shapes run k_conv3x3_fwd.
 template <int CIN>
 bool conv_tile(idmx_ctx_s* c, const void* in, const void* wt, const float* bias, void* out,
-               float* out_f32, const ConvShape& s, int relu, hipError_t& e) {
+               float* out_f32, const ConvShape& s, int relu, const BwdWSum& t, hipError_t& e) {
   constexpr int M = ConvTile<CIN>::CTMAX;
   constexpr size_t LIM = 96 * 1024;
   const int P = s.N * s.H * s.W, cots = (s.Cout + 15) / 16;
@@ -523,25 +526,36 @@ bool conv_tile(idmx_ctx_s* c, const void* in, const void* wt, const float* bias,
   const int tp = big ? 256 : 64;
   if (ConvTile<CIN>::lds(s.W, tp) > LIM) return false;
   while (ct > 1 && (int64_t)(P + tp - 1) / tp * (cots / ct) < 512) ct /= 2;
-  e = big ? conv_tile_ct<CIN, 256>(c, in, wt, bias, out, out_f32, s, relu, ct)
-          : conv_tile_ct<CIN, 64>(c, in, wt, bias, out, out_f32, s, relu, ct);
+  e = big ? conv_tile_ct<CIN, 256>(c, in, wt, bias, out, out_f32, s, relu, ct, t)
+          : conv_tile_ct<CIN, 64>(c, in, wt, bias, out, out_f32, s, relu, ct, t);
   return true;
 }
 
+hipError_t launch_bwd_w_sum(idmx_ctx_s* c, const BwdWSum& t) {
+  hipLaunchKernelGGL(k_conv_bwd_w_sum, dim3((t.n + 63) / 64), dim3(256), 0, c->stream, t);
+  return hipGetLastError();
+}
+
+// With t.part the launch also adds up that weight gradient (a layer's
+// backward-data pass).
 hipError_t conv_fwd(idmx_ctx_s* c, const void* in, const void* wt, const float* bias, void* out,
-                    float* out_f32, const ConvShape& s, int relu) {
+                    float* out_f32, const ConvShape& s, int relu, const BwdWSum& t = {}) {
   hipError_t e = hipSuccess;
   if (aligned(in, 16) && aligned(wt, 8) && aligned(out, 8) && aligned(bias, 16) &&
       aligned(out_f32, 16)) {
     bool done = false;
     switch (s.Cin) {
-      case 8: done = conv_tile<8>(c, in, wt, bias, out, out_f32, s, relu, e); break;
-      case 16: done = conv_tile<16>(c, in, wt, bias, out, out_f32, s, relu, e); break;
-      case 32: done = conv_tile<32>(c, in, wt, bias, out, out_f32, s, relu, e); break;
-      case 64: done = conv_tile<64>(c, in, wt, bias, out, out_f32, s, relu, e); break;
-      case 128: done = conv_tile<128>(c, in, wt, bias, out, out_f32, s, relu, e); break;
+      case 8: done = conv_tile<8>(c, in, wt, bias, out, out_f32, s, relu, t, e); break;
+      case 16: done = conv_tile<16>(c, in, wt, bias, out, out_f32, s, relu, t, e); break;
+      case 32: done = conv_tile<32>(c, in, wt, bias, out, out_f32, s, relu, t, e); break;
+      case 64: done = conv_tile<64>(c, in, wt, bias, out, out_f32, s, relu, t, e); break;
+      case 128: done = conv_tile<128>(c, in, wt, bias, out, out_f32, s, relu, t, e); break;
     }
     if (done) return e;
+  }
+  if (t.part) {
+    e = launch_bwd_w_sum(c, t);
+    if (e != hipSuccess) return e;
   }
   const int64_t waves = (int64_t)((s.N * s.H * s.W + 15) / 16) * ((s.Cout + 15) / 16);
   hipLaunchKernelGGL(k_conv3x3_fwd, dim3(g1(waves * 64)), dim3(256), 0, c->stream,
@@ -552,7 +566,9 @@ hipError_t conv_fwd(idmx_ctx_s* c, const void* in, const void* wt, const float* 
 
 // One layer's weight gradient: its operands, and with y the ReLU mask of dy
 // (in place), with wd the backward-data weights from w, written by the same
-// launches where the tiled kernels apply.
+// launch where the tiled kernels apply; with `later` the sums over the tiled
+// kernel's parts are left to the caller's next launch (*later, before the
+// parts are written again), which has nothing to do if later->part is null.
 struct BwdWArgs {
   const void* in;
   void* dy;
@@ -560,6 +576,7 @@ struct BwdWArgs {
   float *dw, *db;
   const float* w;
   void* wd;
+  BwdWSum* later = nullptr;
 };
 
 template <int CIN, int COUT, int TPX>
@@ -581,14 +598,21 @@ bool bwd_w_run(idmx_ctx_s* c, const BwdWArgs& a, const ConvShape& s, hipError_t&
     if (e != hipSuccess) return true;
     c->nn_part_cap = need;
   }
-  hipLaunchKernelGGL((k_conv3x3_bwd_w_tile<CIN, COUT, TPX>), dim3(blocks), dim3(256),
-                     B::lds(s.W), c->stream, (const uint16_t*)a.in, (uint16_t*)a.dy,
-                     (const uint16_t*)a.y, c->nn_part, s, nchunks);
   const int flips = a.wd ? (nw + 255) / 256 : 0;
-  hipLaunchKernelGGL(k_conv_bwd_w_sum, dim3((nw + COUT + 63) / 64 + flips), dim3(256), 0,
-                     c->stream, c->nn_part, a.dw, a.db, nw, COUT, blocks, a.w, (uint16_t*)a.wd,
-                     CIN, COUT);
+  hipLaunchKernelGGL((k_conv3x3_bwd_w_tile<CIN, COUT, TPX>), dim3(blocks + flips), dim3(256),
+                     B::lds(s.W), c->stream, (const uint16_t*)a.in, (uint16_t*)a.dy,
+                     (const uint16_t*)a.y, c->nn_part, s, nchunks, blocks, a.w, (uint16_t*)a.wd);
   e = hipGetLastError();
+  if (e != hipSuccess) return true;
+  BwdWSum t;
+  t.part = c->nn_part;
+  t.dw = a.dw;
+  t.db = a.db;
+  t.nw = nw;
+  t.n = nw + COUT;
+  t.parts = blocks;
+  if (a.later) *a.later = t;
+  else e = launch_bwd_w_sum(c, t);
   return true;
 }
 
@@ -704,10 +728,12 @@ int idmx_nn_conv3x3_bwd(idmx_ctx_t c, const void* in, const void* y, void* dy, c
   NCHECK(c && in && dy && w && dw && (!dx || wd_scratch) && N > 0 && H > 0 && W > 0 && Cin > 0 &&
              Cout > 0,
          "idmx_nn_conv3x3_bwd: invalid argument");
-  IDMX_HIP(bwd_weight(c, {in, dy, y, dw, db, w, dx ? wd_scratch : nullptr},
+  BwdWSum t;
+  IDMX_HIP(bwd_weight(c, {in, dy, y, dw, db, w, dx ? wd_scratch : nullptr, dx ? &t : nullptr},
                       ConvShape{N, H, W, Cin, Cout}));
   if (dx)
-    IDMX_HIP(conv_fwd(c, dy, wd_scratch, nullptr, dx, nullptr, ConvShape{N, H, W, Cout, Cin}, 0));
+    IDMX_HIP(conv_fwd(c, dy, wd_scratch, nullptr, dx, nullptr, ConvShape{N, H, W, Cout, Cin}, 0,
+                      t));
   return IDMX_OK;
 }
 

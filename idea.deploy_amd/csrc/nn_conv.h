@@ -26,6 +26,34 @@ struct ConvShape {
   int N, H, W, Cin, Cout;
 };
 
+// The sums over a weight gradient's parts: dw[i] += sum_b part[b][i] (i < nw),
+// db[i - nw] likewise (db may be null), 64 sums per block, its four waves over
+// a quarter of the parts each, eight loads in flight.
+struct BwdWSum {
+  const float* part = nullptr;
+  float *dw = nullptr, *db = nullptr;
+  int nw = 0, n = 0, parts = 0;
+  int nx = 0;  // in a convolution's launch: its own blocks along x
+};
+__device__ inline void bwd_w_sum(const BwdWSum& t, int block, float* f) {
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6, i = block * 64 + lane;
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (i < t.n) {
+    int b = g;
+    for (; b + 28 < t.parts; b += 32)
+#pragma unroll
+      for (int k = 0; k < 8; k++) v[k] += t.part[(int64_t)(b + 4 * k) * t.n + i];
+    for (; b < t.parts; b += 4) v[0] += t.part[(int64_t)b * t.n + i];
+  }
+  f[threadIdx.x] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  __syncthreads();
+  if (g == 0 && i < t.n) {
+    const float r = (f[lane] + f[64 + lane]) + (f[128 + lane] + f[192 + lane]);
+    if (i < t.nw) t.dw[i] += r;
+    else if (t.db) t.db[i - t.nw] += r;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Forward 3x3 convolution of TP consecutive pixels (in (n, y, x) order) by CT
 // tiles of 16 output channels per block; the arithmetic of k_conv3x3_fwd, in
@@ -50,15 +78,22 @@ struct ConvTile {
   }
 };
 
-template <int CIN, int CT, int TP>
+template <int CIN, int CT, int TP, bool SUM>
 __global__ void __launch_bounds__(256)
 k_conv3x3_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict__ wt,
                const float* __restrict__ bias, uint16_t* __restrict__ out,
-               float* __restrict__ out_f32, ConvShape s, int relu) {
+               float* __restrict__ out_f32, ConvShape s, int relu, BwdWSum t) {
   using C = ConvTile<CIN>;
   constexpr int SD = C::SD, K = 9 * CIN, NM = TP / 64;  // 16-pixel tiles per wave
   constexpr int NSL = (K + 15) / 16;                    // MFMAs along k
   extern __shared__ uint32_t lds[];
+  // SUM, a backward-data launch: the blocks past its own along x add up the
+  // layer's weight gradient (a launch of its own takes 4.4 us: a training step
+  // of 32 images 457 us with them, 390 without)
+  if (SUM && (int)blockIdx.x >= t.nx) {
+    bwd_w_sum(t, (blockIdx.x - t.nx) * gridDim.y + blockIdx.y, (float*)lds);
+    return;
+  }
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int P = s.N * s.H * s.W, W = s.W;
   const int p0 = blockIdx.x * TP;
@@ -196,7 +231,7 @@ k_conv3x3_tile(const uint16_t* __restrict__ in, const uint16_t* __restrict__ wt,
 // Backward-weight: dW[co][tap * CIN + ci] = sum_p dY[p][co] X[p + tap][ci] as
 // an MFMA GEMM whose reduction runs over pixels. A block accumulates chunks of
 // TPX pixels in registers; its sums go to part[block][co * 9 CIN + k] and are
-// added up by k_conv_bwd_w_sum.
+// added up by bwd_w_sum.
 //
 // The MFMA wants 4 consecutive pixels of one channel per lane, so both
 // operands are staged transposed: X as [ci][row][x] with two zero pixels on
@@ -239,15 +274,27 @@ __device__ __forceinline__ v4u32 relu_mask(v4u32 y, v4u32 g) {
 __device__ __forceinline__ uint32_t mid16(uint32_t a, uint32_t b) { return (a >> 16) | (b << 16); }
 
 // With y (the layer's ReLU output) dY is masked by y > 0 first, in place: a
-// block stages every channel of its pixels, each exactly once.
+// block stages every channel of its pixels, each exactly once. The blocks past
+// the first `blocks` write the weights for the backward-data pass instead, the
+// transposed, tap-flipped kernel wd[ci][tap' Cout + co] =
+// w[co][(8 - tap') Cin + ci] in bf16.
 template <int CIN, int COUT, int TPX>
 __global__ void __launch_bounds__(256)
 k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, uint16_t* __restrict__ dy,
                      const uint16_t* __restrict__ y, float* __restrict__ part, ConvShape s,
-                     int nchunks) {
+                     int nchunks, int blocks, const float* __restrict__ w,
+                     uint16_t* __restrict__ wd) {
   using B = BwdW<CIN, COUT, TPX>;
   constexpr int NI = B::NI, NO = B::NO, YP = B::YP;
   extern __shared__ uint32_t lds[];
+  if ((int)blockIdx.x >= blocks) {
+    const int i = (blockIdx.x - blocks) * 256 + threadIdx.x;
+    if (i < COUT * 9 * CIN) {
+      const int ci = i / (9 * COUT), rem = i % (9 * COUT), tp = rem / COUT, co = rem % COUT;
+      wd[i] = f2bf(w[(int64_t)co * 9 * CIN + (8 - tp) * CIN + ci]);
+    }
+    return;
+  }
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int W = s.W, H = s.H, P = s.N * H * W;
   const int rw = (W + 4) / 2, nrows = TPX / W + 2, plane = ((nrows * rw) + 7) / 8 * 8 + 4;
@@ -273,7 +320,7 @@ k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, uint16_t* __restrict__ dy,
       for (int o = 0; o < NO; o++) acc[i][t / 3][t % 3][o] = {0.f, 0.f, 0.f, 0.f};
   float bsum = 0.f;
 
-  for (int ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
+  for (int ch = blockIdx.x; ch < nchunks; ch += blocks) {
     const int p0 = ch * TPX, row0 = p0 / W - 1;
     __syncthreads();
     // X: 4 pixels x 8 channels per thread and round, transposed in registers
@@ -426,42 +473,9 @@ k_conv3x3_bwd_w_tile(const uint16_t* __restrict__ in, uint16_t* __restrict__ dy,
         }
 }
 
-// dw[i] += sum_b part[b][i] (i < nw), db[i - nw] likewise (db may be null): 64
-// sums per block, its four waves over a quarter of the parts each, eight loads
-// in flight. The blocks past those (fl of them) write the weights for the
-// backward-data pass instead, the transposed, tap-flipped kernel
-// wd[ci][tap' Cout + co] = w[co][(8 - tap') Cin + ci] in bf16.
-__global__ void __launch_bounds__(256)
-k_conv_bwd_w_sum(const float* __restrict__ part, float* __restrict__ dw, float* __restrict__ db,
-                 int nw, int nb, int blocks, const float* __restrict__ w,
-                 uint16_t* __restrict__ wd, int Cin, int Cout) {
-  const int n = nw + nb, sums = (n + 63) / 64;
-  if ((int)blockIdx.x >= sums) {
-    const int i = (blockIdx.x - sums) * 256 + threadIdx.x;
-    if (i < nw) {
-      const int ci = i / (9 * Cout), rem = i % (9 * Cout);
-      const int tp = rem / Cout, co = rem % Cout;
-      wd[i] = f2bf(w[(int64_t)co * 9 * Cin + (8 - tp) * Cin + ci]);
-    }
-    return;
-  }
-  const int i = blockIdx.x * 64 + (threadIdx.x & 63), g = threadIdx.x >> 6;
-  __shared__ float f[4][64];
-  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (i < n) {
-    int b = g;
-    for (; b + 28 < blocks; b += 32)
-#pragma unroll
-      for (int k = 0; k < 8; k++) v[k] += part[(int64_t)(b + 4 * k) * n + i];
-    for (; b < blocks; b += 4) v[0] += part[(int64_t)b * n + i];
-  }
-  f[g][threadIdx.x & 63] = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-  __syncthreads();
-  if (g == 0 && i < n) {
-    const float t = (f[0][threadIdx.x] + f[1][threadIdx.x]) + (f[2][threadIdx.x] + f[3][threadIdx.x]);
-    if (i < nw) dw[i] += t;
-    else if (db) db[i - nw] += t;
-  }
+__global__ void __launch_bounds__(256) k_conv_bwd_w_sum(BwdWSum t) {
+  __shared__ float f[256];
+  bwd_w_sum(t, blockIdx.x, f);
 }
 
 }  // namespace idmx
