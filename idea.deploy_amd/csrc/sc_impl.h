@@ -73,8 +73,9 @@ struct Impl {
 
   // Lead plane staged in LDS by DMA (variant 9); tiles whose staging buffer
   // does not fit the LDS of a CU are refused.
-  template <int TX, int TY, bool XSH = false>
-  static hipError_t launch_dma(idmx_sc_s* s, const T* pop, T* swap) {
+  template <int TX, int TY, bool XSH = false, bool WF = false>
+  static hipError_t launch_dma(idmx_sc_s* s, const T* pop, T* swap, double* n = nullptr,
+                               double* psi = nullptr, double* u = nullptr) {
     if constexpr (DmaShape<S, ES, T, TX, TY, COLL>::fits) {
       const Geom& g = s->geo;
       const int ntx = (g.L0 + TX - 1) / TX;
@@ -84,9 +85,9 @@ struct Impl {
       const int nseg = (Lm + H - 1) / H;
       const int ntiles = ntx * nty * nseg;
       const unsigned grid = (unsigned)((ntiles + 7) / 8 * 8);
-      hipLaunchKernelGGL((k_fused_dma<S, ES, T, SHIFT, COLL, TX, TY, false, XSH>), dim3(grid),
+      hipLaunchKernelGGL((k_fused_dma<S, ES, T, SHIFT, COLL, TX, TY, false, XSH, WF>), dim3(grid),
                          dim3(TX * TY), 0, s->ctx->stream, pop, swap, g, phys(s), H, ntx, nty,
-                         ntiles, nullptr, nullptr, T(0), T(0), T(0), XSH ? s->xsh : 0);
+                         ntiles, nullptr, nullptr, T(0), T(0), T(0), XSH ? s->xsh : 0, n, psi, u);
       return hipGetLastError();
     } else {
       return hipErrorInvalidConfiguration;
@@ -387,6 +388,28 @@ struct Impl {
     }
   }
 
+  // The 3D step that writes n / psi / u, on the LDS-staged step with the run's
+  // own tile: where the rule of the default launch takes that step (20 steps of
+  // 256^3 MRT, the last of them writing the fields: 22.2 ms with registers in
+  // that one, 21.6 here; FP32 11.2 and 10.96).
+  static constexpr bool kDmaWF = S::D == 3 && (COLL == 0 || COLL == 2 || COLL == 3) &&
+                                 (ES::R == 1 || (sizeof(T) == 4 && COLL != 3)) &&
+                                 DmaShape<S, ES, T, 64, 4, COLL>::fits &&
+                                 DmaShape<S, ES, T, 32, 8, COLL>::fits;
+  static bool dma_wf(const idmx_sc_s* s) {
+    return kDmaWF && (COLL == 3 || (s->hist == 10 && (s->tx == 64 || s->tx == 32)));
+  }
+  static hipError_t fused_dma_wf(idmx_sc_s* s, const T* pop, T* swap, double* n, double* psi,
+                                 double* u) {
+    if constexpr (kDmaWF) {
+      if constexpr (COLL != 3)
+        if (s->tx == 32) return launch_dma<32, 8, true, true>(s, pop, swap, n, psi, u);
+      return launch_dma<64, 4, true, true>(s, pop, swap, n, psi, u);
+    } else {
+      return hipErrorInvalidConfiguration;
+    }
+  }
+
   // Tile shapes the autotuner chooses from; the step that writes n/psi/u at
   // a checkpoint uses one fixed shape.
   template <bool WF>
@@ -516,8 +539,8 @@ struct Impl {
     // variant 10, the fused step with walls and the fixed Shan-Chen-forcing /
     // isotropy-filter launch keep the populations in the x-shifted storage
     // between their steps (k_fused_dma<..., XSH>): the first of the nxsh
-    // steps reads the streamed storage, the last writes it (the step that
-    // writes n/psi/u runs on the streamed storage), so a run of one step
+    // steps reads the streamed storage, the last writes it (a step that writes
+    // n/psi/u with registers runs on the streamed storage), so a run of one step
     // never leaves it
     // (small 2D lattices stay on the streamed storage on variant 10: several
     // steps per launch on tiles, single steps with registers)
@@ -527,7 +550,8 @@ struct Impl {
                         s->geo.V < (sizeof(T) == 4 ? kTile3Sites32 : kTile3Sites);
     const bool xs = !small3 && (fwalls || (COLL < 3 ? s->hist == 10 && !small
                                                     : (kFixedDma2 || kFixedDma3)));
-    const int nxsh = xs && !twop ? nsteps - (wf ? 1 : 0) : 0;
+    const bool dwf = wf && xs && !fwalls && dma_wf(s);
+    const int nxsh = xs && !twop ? nsteps - (wf && !dwf ? 1 : 0) : 0;
     if constexpr (COLL < 3) if (pull) {
       hipLaunchKernelGGL((k_restream<S, T>), dim3(grid_for(s->geo.V)), dim3(256), 0, st,
                          (const T*)*pop, (T*)*swap, s->geo, 1);
@@ -597,7 +621,8 @@ struct Impl {
         } else {
           if (mid) IDMX_HIP(hipEventRecord(mid, st));
           s->xsh = k < nxsh ? (k > 0 ? 1 : 0) | (k < nxsh - 1 ? 2 : 0) : 0;
-          if (wf && last) e = fused_fixed<true>(s, a, b, n, psi, u);
+          if (dwf && last) e = fused_dma_wf(s, a, b, n, psi, u);
+          else if (wf && last) e = fused_fixed<true>(s, a, b, n, psi, u);
           else e = fused_fixed<false>(s, a, b, nullptr, nullptr, nullptr);
           s->xsh = 0;
         }
@@ -612,7 +637,8 @@ struct Impl {
         } else {
           if (mid) IDMX_HIP(hipEventRecord(mid, st));
           s->xsh = k < nxsh ? (k > 0 ? 1 : 0) | (k < nxsh - 1 ? 2 : 0) : 0;
-          if (wf && last) e = fused<true>(s, a, b, n, psi, u);
+          if (dwf && last) e = fused_dma_wf(s, a, b, n, psi, u);
+          else if (wf && last) e = fused<true>(s, a, b, n, psi, u);
           else if (small && s->hist == 10) e = fused_regs(s, a, b);
           else e = fused<false>(s, a, b, nullptr, nullptr, nullptr);
           s->xsh = 0;

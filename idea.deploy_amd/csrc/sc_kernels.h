@@ -1050,13 +1050,15 @@ __device__ __forceinline__ void dma_dword(uint64_t base, uint32_t voff, uint32_t
 // body force (bx, by, bz) added to the Shan-Chen force: psi_w is the psi
 // array (its non-fluid sites are staged with the populations), wmask the
 // per-site masks (kWallSelf). FP64 only.
+// WF: also writes n, psi and u of the step.
 template <class S, class ES, class T, bool SHIFT, int COLL, int TX, int TY, bool WALLS = false,
-          bool XSH = false>
+          bool XSH = false, bool WF = false>
 __global__ void __launch_bounds__(TX * TY)
 k_fused_dma(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> P, int H,
             int ntx, int nty, int ntiles, const double* __restrict__ psi_w = nullptr,
             const uint64_t* __restrict__ wmask = nullptr, T bx = T(0), T by = T(0),
-            T bz = T(0), int xsh = 0) {
+            T bz = T(0), int xsh = 0, double* __restrict__ n_out = nullptr,
+            double* __restrict__ psi_out = nullptr, double* __restrict__ u_out = nullptr) {
   using SH = DmaShape<S, ES, T, TX, TY, COLL, WALLS>;
   constexpr int D = S::D, Q = S::Q, R = ES::R;
   constexpr int NT = SH::NT, PX = SH::PX, PY = SH::PY, NP = SH::NP, NS = SH::NS;
@@ -1332,6 +1334,14 @@ k_fused_dma(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<
         collide<S, T, SHIFT, COLL, WALLS>(fh[0], dnh[0], gx, gy, gz, lpsi, PL, fpend, u, bx, by,
                                           bz);
         if constexpr (WALLS) pend_mask = mh[0];
+        if constexpr (WF) {
+          const int64_t g = (int64_t)mc * PS + (int64_t)y * geo.L0 + x;
+          n_out[g] = (double)(SHIFT ? P.rho0 + dnh[0] : dnh[0]);
+          psi_out[g] = (double)lpsi;
+          u_out[g] = (double)u[0];
+          u_out[g + geo.V] = (double)u[1];
+          if (D == 3) u_out[g + 2 * geo.V] = (double)u[2];
+        }
       }
       pend_m = m0 + j - 2 * R;
     }
