@@ -187,10 +187,10 @@ int idmx_batch_create(idmx_ctx_t ctx, const idmx_batch_domain* doms, int ndom, i
   hipGetDeviceProperties(&p, ctx->device);
   b->grid = p.multiProcessorCount * 8;
   // With the E4 force two steps per launch on the x-shifted storage (64
-  // domains of 64^2 to 256^2, FP64: 42.8 us per step with 16 x 16 tiles, 73.2
+  // domains of 64^2 to 256^2, FP64: 39.4 us per step with 16 x 16 tiles, 73.2
   // with the one-step 32 x 8 ones; one domain of 128^2: 3.3 against 4.1).
   // FP32 keeps three blocks of 32 x 16 per CU, which re-read less, as long as
-  // there are enough of them (22.0 against 24.2 us at 32 x 8).
+  // there are enough of them (20.5 against 22.0 us at 32 x 8).
   if (estencil == IDMX_E4) {
     b->kind = 5;
     const bool wide = precision == IDMX_PREC_F32S && so >= 200000;

@@ -37,8 +37,8 @@ struct idmx_batch_s {
   int grid = 0;
   // no idmx_batch_set_launch yet with a grid: a step launch has one block per
   // live item, which the dispatcher balances better than blocks striding over
-  // the items (64 domains of 64^2 to 256^2, kind 5: 42.8 us per step against
-  // 48.5 with 2048 blocks; E8, kind 1: 69.8 against 76.2)
+  // the items (64 domains of 64^2 to 256^2, kind 5: 39.4 us per step against
+  // 44.1 with 2048 blocks; E8, kind 1: 69.8 against 76.2)
   bool grid_auto = true;
   hipGraphExec_t graph = nullptr;
   int graph_steps = 0;

@@ -8,7 +8,9 @@
 // Tensors are NHWC. Activations and weights used by the MFMA are bf16
 // (stored as uint16 bit patterns); master weights, gradients and the loss
 // are FP32. Conv weights are [Cout][9*Cin] with k = tap*Cin + ci,
-// tap = 3*ky + kx. When Cin is a multiple of 4 a lane's MFMA K slice is 4
+// tap = 3*ky + kx. Layers of 8, 16, 32, 64 or 128 channels run the tiled
+// kernels of nn_conv.h, the convolutions here take the other shapes: when
+// Cin is a multiple of 4 a lane's MFMA K slice is 4
 // channels of one tap (vector loads); other channel counts are handled
 // element by element.
 #include <hip/hip_runtime.h>
@@ -595,7 +597,11 @@ bool bwd_w_run(idmx_ctx_s* c, const BwdWArgs& a, const ConvShape& s, hipError_t&
     c->nn_part = nullptr;
     c->nn_part_cap = 0;
     e = hipMalloc(&c->nn_part, need * sizeof(float));
-    if (e != hipSuccess) return true;
+    if (e != hipSuccess) {  // no room: the kernel that needs no workspace
+      (void)hipGetLastError();
+      c->nn_part = nullptr;
+      return false;
+    }
     c->nn_part_cap = need;
   }
   const int flips = a.wd ? (nw + 255) / 256 : 0;

@@ -2,12 +2,12 @@
 // populations (the single-domain step on the x-shifted storage, 2D).
 //
 // What bounds it: a single step is bound by HBM (144 B per site and step in
-// FP64); two steps per pass halve that, and the FP64 vector units and the
-// latency of two waves per SIMD take over (4096^2 E8: vector units issuing in
-// 60 % of the cycles, 4.6 TB/s). Measured per step on one MI355X, against the
-// best single-step launch: 4096^2 E8 316 us (532), 4096^2 E4 286 us (520),
-// 1000 x 613 Shan-Chen forcing 15 us (30), 1024^2 MRT 23 us (38.5), 4096^2
-// FP32 239 us (270).
+// FP64); two steps per pass move 86 (4096^2 E8, measured), and the FP64 vector
+// units and the latency of two waves per SIMD take over (vector units issuing
+// in 54 % of the cycles, 4.6 TB/s). Measured per step on one MI355X, against
+// the best single-step launch: 4096^2 E8 306 us (532), 4096^2 E4 291 us (520),
+// 1000 x 613 Shan-Chen forcing 13.7 us (30), 1024^2 MRT 23 us (38.5), 4096^2
+// FP32 161 us (270).
 //
 // Layout: a block of NT threads owns a strip of NT columns, of which the
 // inner TXMAX or fewer are written, and marches along y; a thread keeps its
@@ -54,7 +54,7 @@ struct PairShape {
 // geo.L1 rows by H per block, txo columns written per block; xsh as in
 // k_fused_dma (bit 0: reads the x-shifted storage, bit 1: writes it); WF: the
 // second step also writes n, psi and u. Compiled for two waves per SIMD: at
-// three the E4 step spills and runs at 296 us (4096^2) instead of 286.
+// three the E4 step spills (4096^2, at an earlier state: 296 us instead of 286).
 // WALLS: as in k_fused_dma; psi_out holds the psi of the solid sites, which
 // stays, wmask the masks.
 template <class ES, class T, bool SHIFT, int COLL, int NT, bool WF, bool WALLS = false>

@@ -306,10 +306,12 @@ int idmx_sc_pop_from_f64(idmx_sc_t sim, void* pop, const double* src_dev);
  * at x - c_qx, so every push store is line-aligned; the run's first step
  * reads the streamed storage and its last writes it, so pop holds streamed
  * populations between calls, and the results equal variant 9's bit for
- * bit; in 2D a run on variant 10 takes two steps per launch from 3 * 2^17
- * sites up, and four below that with the E4 force, with tiles of its own: tx
- * and H then apply to the single steps left over, which below that size hold
- * the populations in registers). Chosen at creation;
+ * bit; in 2D a run on variant 10 takes two steps per launch, or four on small
+ * lattices with the E4 force, with tiles of its own: tx and H then apply to
+ * the single steps left over, which below 2^19 sites (E6 / E8 in FP64 3 *
+ * 2^17) hold the populations in registers). Chosen at creation, where 3D
+ * lattices below 150000 sites (FP32 100000) get a step without a march that
+ * no variant names;
  * the autotuner (idmx.tune) overrides it. No reference counterpart: the
  * reference fixes block = 128 threads (idpy/LBM/MultiPhase.py:2072-2085). */
 int idmx_sc_set_launch(idmx_sc_t sim, int tx, int ty, int H, int hist);
