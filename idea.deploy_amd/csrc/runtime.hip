@@ -412,23 +412,29 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
     const int blocks_at_8 = ntx * nty * ((Lm + 7) / 8);
     H = std::max(H, blocks_at_8 >= 256 ? 8 : (D == 2 ? 1 : 2));
     s->H = std::min(H, Lm);
-    // 3D lattices that fill the chip: the LDS-staged step on the x-shifted
-    // storage, with the tile and H of the least total (march_planes; one full
-    // round where the lattice allows it: 150 x 101 x 93 127 us per step at
-    // 32 x 8, H = 14, 455 blocks, against 142 at H = 8; 200^3 MRT 592 us at
-    // 64 x 4, H = 40, against 816 with registers). A plane of 32 x 8 takes 6 % longer than one of 64 x 4 (shorter rows), but
-    // pads less on most widths. Reach-2 stencils in FP64 leave one block per
-    // CU and stay on registers (96^3 E8: 86 us against 131), as does the dense
-    // MRT collision, which is bound by its 741 products (128^3: 503 us against
+    // 3D: two blocks share a CU, and the tile and H with the least total win
+    // (march_planes; one full round where the lattice allows it). Against the
+    // segments above, with registers: 65 x 50 x 117 E8 MRT 58 us per step (84),
+    // 96^3 E8 78 (83), 98 x 72 x 205 E8 152 (185), 69 x 93 x 58 E8 FP32 32
+    // (43), dense MRT 128^3 465 (498). A plane of 32 x 8 takes 6 % longer than
+    // one of 64 x 4 (shorter rows), but pads less on most widths.
+    // Lattices that fill the chip run the LDS-staged step on the x-shifted
+    // storage (150 x 101 x 93 127 us per step at 32 x 8, H = 14, against 142
+    // at H = 8; 200^3 MRT 592 us at 64 x 4, H = 40, against 816 with
+    // registers). Reach-2 stencils in FP64 leave one of its blocks per CU and
+    // stay on registers (96^3 E8: 78 us against 131), as does the dense MRT
+    // collision, which is bound by its 741 products (128^3: 465 us against
     // 556) and lattices of a few planes per block (48 x 44 x 40: 14.2 us
     // against 17.4; 64^3 FP32: 14.1 against 15.4).
     const bool f32 = d->precision == IDMX_PREC_F32S;
-    if (D == 3 && (R == 1 || f32) && s->coll != 1 && V >= (f32 ? 500000 : 200000)) {
+    if (D == 3 && !(s->coll == 3 && R == 2)) {
+      const bool staged =
+          (R == 1 || f32) && s->coll != 1 && V >= (f32 ? 500000 : 200000);
       double least = 1e300;
       for (int tx : {64, 32}) {
         const int ty = 256 / tx;
         // the Shan-Chen forcing runs 64 x 4 tiles (Impl::fused_fixed)
-        if ((tx == 32 && s->coll == 3) || !s->ops->launch_ok(tx, ty, 10)) continue;
+        if ((tx == 32 && s->coll == 3) || (staged && !s->ops->launch_ok(tx, ty, 10))) continue;
         const int64_t tiles =
             (int64_t)((s->geo.L0 + tx - 1) / tx) * ((s->geo.L1 + ty - 1) / ty);
         double c;
@@ -439,7 +445,7 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
           s->tx = tx;
           s->ty = ty;
           s->H = h;
-          s->hist = 10;
+          if (staged) s->hist = 10;
         }
       }
     }
