@@ -387,12 +387,12 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
     set_error("idmx_sc_create: unsupported combination");
     return IDMX_E_UNSUPPORTED;
   }
-  // Fused launch shape: rows of 256 (or 64) in 2D, 32 x 8 tiles in 3D; march
-  // segments sized to give >= 2048 blocks where the lattice allows it, and
-  // at least 8 planes long unless that leaves fewer than 256 blocks: on
-  // small lattices a block's march is a chain of dependent plane steps, so
-  // short segments run faster (measured per step: 128^2 15.2 us at 8 planes,
-  // 5.6 us at 1; 64^3 41.4 us at 8, 24.7 us at 2; 96^3 and up best at 8).
+  // Fused launch shape of single steps: rows of 256 (or 64) in 2D, 32 x 8 tiles
+  // in 3D until the rule further down; march segments sized to give >= 2048
+  // blocks where the lattice allows it, and at least 8 planes long unless that
+  // leaves fewer than 256 blocks: on small lattices a block's march is a chain
+  // of dependent plane steps, so short segments run faster (measured per step:
+  // 128^2 15.2 us at 8 planes, 5.6 us at 1).
   if (D == 2) {
     s->tx = d->dims[0] >= 256 ? 256 : 64;
     s->ty = 1;
