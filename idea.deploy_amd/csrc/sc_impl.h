@@ -473,12 +473,13 @@ struct Impl {
     // step of its own that writes n / psi / u is the two-pass one (from 2^19
     // sites up, or when asked for: on smaller lattices two passes are as
     // fast as single fused steps; measured 0.94x at 64^3, 1.07x at 1024^2,
-    // 1.30x at 256^3 and 1.47x at 4096^2)
-    const bool fwalls = kFusedWalls && s->walls && (flags & IDMX_RUN_TWO_PASS) == 0 &&
-                        s->desc.psi_kind != IDMX_PSI_PROGRAM &&
-                        (s->geo.V >= (int64_t(1) << 19) || (flags & IDMX_RUN_FUSED_WALLS) != 0);
-    const bool twop = !fwalls && ((flags & IDMX_RUN_TWO_PASS) != 0 || s->walls || body ||
-                                  s->desc.psi_kind == IDMX_PSI_PROGRAM);
+    // 1.30x at 256^3 and 1.47x at 4096^2). With a flag that is neither 0 nor
+    // 1 the steps after the first launch are two-pass ones as well.
+    bool fwalls = kFusedWalls && s->walls && (flags & IDMX_RUN_TWO_PASS) == 0 &&
+                  s->desc.psi_kind != IDMX_PSI_PROGRAM &&
+                  (s->geo.V >= (int64_t(1) << 19) || (flags & IDMX_RUN_FUSED_WALLS) != 0);
+    bool twop = !fwalls && ((flags & IDMX_RUN_TWO_PASS) != 0 || s->walls || body ||
+                            s->desc.psi_kind == IDMX_PSI_PROGRAM);
     if ((twop || fwalls) && (!n || !psi)) {
       set_error(s->walls || body || s->desc.psi_kind == IDMX_PSI_PROGRAM
                     ? "idmx_sc_run: walls, a body force or a psi program need the n and psi "
@@ -510,9 +511,11 @@ struct Impl {
         set_error("idmx_sc_run: wall masks not allocated (idmx_sc_set_walls)");
         return IDMX_E_NOMEM;
       }
+      *s->wflag_host = 0;
       hipLaunchKernelGGL((k_wall_mask<S>), dim3(grid_for(s->geo.V)), dim3(256), 0, st, s->walls,
-                         s->geo, s->wmask_dev, (uint32_t*)nullptr);
+                         s->geo, s->wmask_dev, s->wflag_host);
       IDMX_HIP(hipGetLastError());
+      IDMX_HIP(hipEventRecord(s->ctx->ev1, st));
     }
     // smaller 2D lattices with walls: several steps per launch, if every flag
     // is 0 or 1 (waiting for that costs 10 us; a run of 8 steps of 128^2
@@ -561,13 +564,48 @@ struct Impl {
     // two steps per launch: an even number of pairs, so that the state ends in
     // the buffer in which single steps would leave it
     const PairPlan pp = S::D == 2 && xs && !twop && !pev ? pair_plan(s, fwalls) : PairPlan{};
-    const int npair = pp.nt ? nsteps / 2 & ~1 : 0;
+    int npair = pp.nt ? nsteps / 2 & ~1 : 0, k0 = 0;
+    // With walls the first launch (the run's single steps come first, then its
+    // pairs) stays on the streamed storage, and while it runs the host learns
+    // from k_wall_mask whether every flag is 0 or 1. If not, the slots that
+    // nothing streams into keep their values of two steps before, which neither
+    // the pairs nor the x-shifted storage can leave in place: two-pass steps
+    // follow. A first single step is then right as it is (its slots are the
+    // two-pass step's); a pair is taken as not done: it has written only
+    // slots that the first of those steps writes again.
+    if constexpr (kFusedWalls) if (fwalls && nsteps > 0 && !(wf && nsteps == 1)) {
+      const bool two = npair > 0 && 2 * npair == nsteps;
+      const T* a = (const T*)*pop;
+      T* b = (T*)*swap;
+      if (pev) {
+        IDMX_HIP(hipEventRecord(pev[0], st));
+        IDMX_HIP(hipEventRecord(pev[1], st));
+      }
+      s->xsh = 0;
+      const hipError_t e = two ? pair(s, pp, true, a, b, nullptr, psi, u)
+                               : fused_walls(s, a, b, psi);
+      if (e != hipSuccess) return hip_fail(e, "idmx_sc_run launch");
+      if (nsteps > 1) IDMX_HIP(hipEventSynchronize(s->ctx->ev1));
+      if (nsteps > 1 && *s->wflag_host) {
+        fwalls = false;
+        twop = true;
+        npair = 0;
+        if (!two) k0 = 1;
+      } else {
+        k0 = 1;
+      }
+      if (k0) std::swap(*pop, *swap);
+    }
+    // storage of the k-th launch of n on the x-shifted storage
+    auto shift = [&](int k, int n) {
+      return (k > (fwalls ? 1 : 0) ? 1 : 0) | (k < n - 1 ? 2 : 0);
+    };
     if (npair > 0) {
       const int nl = nsteps - npair;  // single steps first, then the pairs
-      for (int k = 0; k < nl; k++) {
+      for (int k = k0; k < nl; k++) {
         const T* a = (const T*)*pop;
         T* b = (T*)*swap;
-        s->xsh = (k > 0 ? 1 : 0) | (k < nl - 1 ? 2 : 0);
+        s->xsh = shift(k, nl);
         const bool f = wf && k == nl - 1;
         hipError_t e;
         if (k >= nl - npair) e = pair(s, pp, fwalls, a, b, f ? n : nullptr, psi, u);
@@ -602,7 +640,7 @@ struct Impl {
           std::swap(*pop, *swap);
         }
       }
-    for (int k = npair > 0 || nquad > 0 ? nsteps : 0; k < nsteps; k++) {
+    for (int k = npair > 0 || nquad > 0 ? nsteps : k0; k < nsteps; k++) {
       const bool last = k == nsteps - 1;
       const T* a = (const T*)*pop;
       T* b = (T*)*swap;
@@ -620,7 +658,7 @@ struct Impl {
           e = two_pass(s, a, b, n, psi, u, wf && last, mid);
         } else {
           if (mid) IDMX_HIP(hipEventRecord(mid, st));
-          s->xsh = k < nxsh ? (k > 0 ? 1 : 0) | (k < nxsh - 1 ? 2 : 0) : 0;
+          s->xsh = k < nxsh ? shift(k, nxsh) : 0;
           if (dwf && last) e = fused_dma_wf(s, a, b, n, psi, u);
           else if (wf && last) e = fused_fixed<true>(s, a, b, n, psi, u);
           else e = fused_fixed<false>(s, a, b, nullptr, nullptr, nullptr);
@@ -631,12 +669,12 @@ struct Impl {
           e = two_pass(s, a, b, n, psi, u, wf && last, mid);
         } else if (fwalls) {
           if (mid) IDMX_HIP(hipEventRecord(mid, st));
-          s->xsh = k < nxsh ? (k > 0 ? 1 : 0) | (k < nxsh - 1 ? 2 : 0) : 0;
+          s->xsh = k < nxsh ? shift(k, nxsh) : 0;
           e = fused_walls(s, a, b, psi);
           s->xsh = 0;
         } else {
           if (mid) IDMX_HIP(hipEventRecord(mid, st));
-          s->xsh = k < nxsh ? (k > 0 ? 1 : 0) | (k < nxsh - 1 ? 2 : 0) : 0;
+          s->xsh = k < nxsh ? shift(k, nxsh) : 0;
           if (dwf && last) e = fused_dma_wf(s, a, b, n, psi, u);
           else if (wf && last) e = fused<true>(s, a, b, n, psi, u);
           else if (small && s->hist == 10) e = fused_regs(s, a, b);

@@ -1026,8 +1026,7 @@ struct DmaShape {
 // Wall mask of a site for the fused steps with walls: bit q (q >= 1) when the
 // neighbour x + c_q is solid (flag 0: the population pushed there bounces
 // back), bit 0 when the site itself is not fluid (flag != 1: not updated, its
-// psi is the one the caller stored), bit Q + q when the neighbour x - c_q is
-// neither (nothing streams in from there).
+// psi is the one the caller stored).
 constexpr int kWallSelf = 0;
 
 __device__ __forceinline__ void lds_barrier() {
@@ -1439,7 +1438,7 @@ __device__ inline void site_xyz(const Geom& geo, int64_t g, int& x, int& y, int&
 
 // The per-site wall masks of the fused step with walls (kWallSelf), from the
 // flags: recomputed at every run, so flags changed between runs are seen.
-// Writes 1 to *other (unless null) when a flag is neither 0 nor 1.
+// Writes 1 to *other when a flag is neither 0 nor 1.
 template <class S>
 __global__ void __launch_bounds__(256)
 k_wall_mask(const uint8_t* __restrict__ walls, Geom geo, uint64_t* __restrict__ mask,
@@ -1448,16 +1447,14 @@ k_wall_mask(const uint8_t* __restrict__ walls, Geom geo, uint64_t* __restrict__ 
        g += (int64_t)gridDim.x * blockDim.x) {
     int x, y, z;
     site_xyz(geo, g, x, y, z);
-    if (other && walls[g] > 1) *other = 1;
+    if (walls[g] > 1) *other = 1;
     uint64_t m = walls[g] != 1 ? (uint64_t(1) << kWallSelf) : uint64_t(0);
 #pragma unroll
     for (int q = 1; q < S::Q; q++) {
       const int xt = S::cx[q] ? wrap(x + S::cx[q], geo.L0) : x;
       const int yt = S::cy[q] ? wrap(y + S::cy[q], geo.L1) : y;
       const int zt = S::cz[q] ? wrap(z + S::cz[q], geo.L2) : z;
-      const uint8_t w = walls[lex(geo, xt, yt, zt)];
-      if (w == 0) m |= uint64_t(1) << q;
-      else if (w != 1) m |= uint64_t(1) << (S::Q + opposite<S>(q));
+      if (walls[lex(geo, xt, yt, zt)] == 0) m |= uint64_t(1) << q;
     }
     mask[g] = m;
   }

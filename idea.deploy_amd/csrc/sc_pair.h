@@ -55,7 +55,8 @@ struct PairShape {
 // k_fused_dma (bit 0: reads the x-shifted storage, bit 1: writes it); WF: the
 // second step also writes n, psi and u. Compiled for two waves per SIMD: at
 // three the E4 step spills (4096^2, at an earlier state: 296 us instead of 286).
-// WALLS: as in k_fused_dma; psi_out holds the psi of the solid sites, which
+// WALLS: as in k_fused_dma, flags 0 and 1 only (with others the results are
+// dropped by Impl::run); psi_out holds the psi of the solid sites, which
 // stays, wmask the masks.
 template <class ES, class T, bool SHIFT, int COLL, int NT, bool WF, bool WALLS = false>
 __global__ void __launch_bounds__(NT, 2)
@@ -200,8 +201,6 @@ k_pair2d(const T* __restrict__ pop, T* __restrict__ pop_swap, Geom geo, Phys<T> 
             const int o = opposite<S>(q);
             if (m >> q & 1) frow[f_base(o) + slot(o, -R)][tid + 1] = fo[q];
             else frow[f_base(q) + slot(q, S::cy[q] - R)][tid + 1 + S::cx[q]] = fo[q];
-            // a population that nothing streams into keeps its value
-            if (m >> (Q + q) & 1) frow[f_base(q) + slot(q, -R)][tid + 1] = fh0[B0][q];
           }
         }
       } else {

@@ -84,7 +84,9 @@ enum {
                                 lattices several steps per launch, where the
                                 run has at least 8, or the two-pass step; a
                                 single last step of a run that writes the
-                                fields is the two-pass one) */
+                                fields is the two-pass one, and so is every
+                                step where a flag is neither 0 nor 1 and more
+                                than one step is taken) */
 };
 
 typedef struct idmx_ctx_s* idmx_ctx_t;
