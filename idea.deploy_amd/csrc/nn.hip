@@ -660,7 +660,10 @@ hipError_t flip_weights(idmx_ctx_s* c, const float* w, void* wd, int Cin, int Co
 
 hipError_t bwd_weight(idmx_ctx_s* c, const BwdWArgs& a, const ConvShape& s) {
   hipError_t e = hipSuccess;
-  if (aligned(a.in, 16) && aligned(a.dy, 16) && aligned(a.y, 16)) {
+  // (no pixels, which idmx_nn_conv3x3_bwd_weight lets pass: nothing to add, and
+  // nothing for the tiled kernels to divide by or to launch)
+  const bool pixels = s.N > 0 && s.H > 0 && s.W > 0;
+  if (pixels && aligned(a.in, 16) && aligned(a.dy, 16) && aligned(a.y, 16)) {
     bool done = false;
     switch (s.Cin) {
       case 8: done = bwd_w_cout<8>(c, a, s, e); break;
