@@ -185,7 +185,7 @@ int idmx_batch_create(idmx_ctx_t ctx, const idmx_batch_domain* doms, int ndom, i
   }
   hipDeviceProp_t p;
   hipGetDeviceProperties(&p, ctx->device);
-  b->grid = p.multiProcessorCount * 8;
+  b->grid = b->first_grid = p.multiProcessorCount * 8;
   // With the E4 force two steps per launch on the x-shifted storage (64
   // domains of 64^2 to 256^2, FP64: 39.4 us per step with 16 x 16 tiles, 73.2
   // with the one-step 32 x 8 ones; one domain of 128^2: 3.3 against 4.1).
@@ -239,7 +239,7 @@ int idmx_batch_set_launch(idmx_batch_t b, int kind, int tx, int H, int grid) {
   b->H = H;
   if (grid > 0) {
     b->grid = grid;
-    b->grid_auto = false;
+    b->grid_auto = grid == b->first_grid;
   }
   drop_graph(b);
   return rebuild_items(b);

@@ -35,11 +35,12 @@ struct idmx_batch_s {
   unsigned long long* d_dmax = nullptr;
   int max_items = 0, n_items = 0;
   int grid = 0;
-  // no idmx_batch_set_launch yet with a grid: a step launch has one block per
-  // live item, which the dispatcher balances better than blocks striding over
+  // the grid is the one of creation, which stands for one block per live item
+  // in a step launch; the dispatcher balances better than blocks striding over
   // the items (64 domains of 64^2 to 256^2, kind 5: 39.4 us per step against
   // 44.1 with 2048 blocks; E8, kind 1: 69.8 against 76.2)
   bool grid_auto = true;
+  int first_grid = 0;
   hipGraphExec_t graph = nullptr;
   int graph_steps = 0;
   int graph_grid = 0;  // step grid the graph was captured with

@@ -71,7 +71,10 @@ struct idmx_sc_s {
   const SimOps* ops = nullptr;
   // fused launch shape (chosen at create time, autotuner may override)
   int tx = 0, ty = 0, H = 0, hist = 1;
-  bool auto_launch = true;  // no idmx_sc_set_launch yet
+  // the launch chosen at creation (tx, ty, H, hist), and whether it is in
+  // force: it includes a step and a march length that the four do not name
+  int first_launch[4] = {0, 0, 0, 0};
+  bool auto_launch = true;
   int xsh = 0;  // variant 10: the running step's x-shifted storage flags
   int coll = 0;  // 0 BGK, 1 dense MRT, 2 diagonal MRT, 3 BGK with Shan-Chen forcing,
                  // 4 BGK followed by the isotropy filter

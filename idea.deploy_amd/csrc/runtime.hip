@@ -477,6 +477,8 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
       return hip_fail(e, "idmx_sc_create: MRT tables");
     }
   }
+  const int first[4] = {s->tx, s->ty, s->H, s->hist};
+  std::copy(first, first + 4, s->first_launch);
   *out = s;
   return IDMX_OK;
 }
@@ -504,24 +506,38 @@ int idmx_sc_pop_bytes(idmx_sc_t s, size_t* bytes) {
   return IDMX_OK;
 }
 
+// Why a launch is not possible, or null.
+static const char* launch_error(const idmx_sc_s* s, int tx, int ty, int H, int hist) {
+  if (s->D == 2) {
+    if (!((tx == 64 || tx == 128 || tx == 256) && ty == 1))
+      return "idmx_sc_set_launch: 2D tiles are 64, 128 or 256 sites wide, ty = 1";
+  } else if (!((tx == 32 && ty == 8) || (tx == 64 && ty == 4) || (tx == 128 && ty == 2) ||
+               (tx == 256 && ty == 2))) {
+    return "idmx_sc_set_launch: 3D tiles are 32x8, 64x4, 128x2 or 256x2";
+  }
+  if (H < 1) return "idmx_sc_set_launch: H must be >= 1";
+  if (hist < 0 || hist > 10) return "idmx_sc_set_launch: variant is 0..10";
+  if (!s->ops->launch_ok(tx, ty, hist))
+    return "idmx_sc_set_launch: the LDS staging of variants 9 and 10 does not fit this tile";
+  return nullptr;
+}
+
+int idmx_sc_launch_ok(idmx_sc_t s, int tx, int ty, int H, int hist, int* ok) {
+  CHECK_ARG(s && ok, "idmx_sc_launch_ok: invalid argument");
+  *ok = launch_error(s, tx, ty, H, hist) == nullptr;
+  return IDMX_OK;
+}
+
 int idmx_sc_set_launch(idmx_sc_t s, int tx, int ty, int H, int hist) {
   CHECK_ARG(s, "idmx_sc_set_launch: null simulation");
-  if (s->D == 2)
-    CHECK_ARG((tx == 64 || tx == 128 || tx == 256) && ty == 1,
-              "idmx_sc_set_launch: 2D tiles are 64, 128 or 256 sites wide, ty = 1");
-  else
-    CHECK_ARG((tx == 32 && ty == 8) || (tx == 64 && ty == 4) || (tx == 128 && ty == 2) ||
-                  (tx == 256 && ty == 2),
-              "idmx_sc_set_launch: 3D tiles are 32x8, 64x4, 128x2 or 256x2");
-  CHECK_ARG(H >= 1, "idmx_sc_set_launch: H must be >= 1");
-  CHECK_ARG(hist >= 0 && hist <= 10, "idmx_sc_set_launch: variant is 0..10");
-  CHECK_ARG(s->ops->launch_ok(tx, ty, hist),
-            "idmx_sc_set_launch: the LDS staging of variants 9 and 10 does not fit this tile");
+  const char* why = launch_error(s, tx, ty, H, hist);
+  CHECK_ARG(!why, why);
   s->tx = tx;
   s->ty = ty;
   s->H = H;
   s->hist = hist;
-  s->auto_launch = false;
+  s->auto_launch = tx == s->first_launch[0] && ty == s->first_launch[1] &&
+                   H == s->first_launch[2] && hist == s->first_launch[3];
   return IDMX_OK;
 }
 

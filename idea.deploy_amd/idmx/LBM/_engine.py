@@ -215,15 +215,11 @@ class SCEngine:
 
     def launch_ok(self, tx, ty, H, hist=1):
         """Whether set_launch accepts this shape (variant 9 needs its LDS
-        staging buffer to fit one CU); the current launch is kept."""
-        old = self.get_launch()
-        try:
-            self.set_launch(tx, ty, H, hist)
-            return True
-        except _lib.IdmxError:
-            return False
-        finally:
-            self.set_launch(*old)
+        staging buffer to fit one CU); nothing is set."""
+        ok = C.c_int()
+        _lib.call('idmx_sc_launch_ok', self.handle, int(tx), int(ty), int(H), int(hist),
+                  C.byref(ok))
+        return bool(ok.value)
 
     def get_launch(self):
         v = [C.c_int() for _ in range(4)]

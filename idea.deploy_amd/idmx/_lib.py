@@ -73,6 +73,7 @@ _SIGS = [
     ('idmx_sc_create', C.c_int, [C.c_void_p, C.POINTER(ScDesc), c_void_pp]),
     ('idmx_sc_destroy', C.c_int, [C.c_void_p]),
     ('idmx_sc_pop_bytes', C.c_int, [C.c_void_p, C.POINTER(C.c_size_t)]),
+    ('idmx_sc_launch_ok', C.c_int, [C.c_void_p] + [C.c_int] * 4 + [C.POINTER(C.c_int)]),
     ('idmx_sc_set_launch', C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int]),
     ('idmx_sc_set_walls', C.c_int, [C.c_void_p, C.c_void_p]),
     ('idmx_sc_set_body_force', C.c_int, [C.c_void_p, C.c_double, C.c_double, C.c_double]),

@@ -313,10 +313,15 @@ int idmx_sc_pop_from_f64(idmx_sc_t sim, void* pop, const double* src_dev);
  * the single steps left over, which below 2^19 sites (E6 / E8 in FP64 3 *
  * 2^17) hold the populations in registers). Chosen at creation, where 3D
  * lattices below 150000 sites (FP32 100000) get a step without a march that
- * no variant names;
+ * no variant names, and 3D steps with walls a march length of their own: what
+ * idmx_sc_get_launch then returns stands for that choice, and setting it
+ * again returns to it;
  * the autotuner (idmx.tune) overrides it. No reference counterpart: the
  * reference fixes block = 128 threads (idpy/LBM/MultiPhase.py:2072-2085). */
 int idmx_sc_set_launch(idmx_sc_t sim, int tx, int ty, int H, int hist);
+/* *ok = 1 where idmx_sc_set_launch accepts this launch, else 0; the present
+ * launch stays. */
+int idmx_sc_launch_ok(idmx_sc_t sim, int tx, int ty, int H, int hist, int* ok);
 
 /* The pseudopotential of a simulation created with IDMX_PSI_PROGRAM: the
  * C expression psi_code that the reference compiles into
@@ -393,7 +398,8 @@ int idmx_batch_destroy(idmx_batch_t b);
  * writes the streamed storage at its ends, and the results equal kind 4's
  * bit for bit. grid = blocks of a step
  * launch (0 keeps the current grid); a step launches at most one block per
- * live work item, and each XCD takes a contiguous run of items. Picked by
+ * live work item, with the grid of creation (8 blocks per CU, as
+ * idmx_batch_get_launch returns it) always that many, and each XCD takes a contiguous run of items. Picked by
  * the autotuner (idmx.tune). */
 int idmx_batch_set_launch(idmx_batch_t b, int kind, int tx, int H, int grid);
 int idmx_batch_get_launch(idmx_batch_t b, int* kind, int* tx, int* H, int* grid,
