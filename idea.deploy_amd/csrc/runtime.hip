@@ -419,7 +419,7 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
     // (43), dense MRT 128^3 465 (498). A plane of 32 x 8 takes 6 % longer than
     // one of 64 x 4 (shorter rows), but pads less on most widths.
     // Lattices that fill the chip run the LDS-staged step on the x-shifted
-    // storage (150 x 101 x 93 127 us per step at 32 x 8, H = 14, against 142
+    // storage (150 x 101 x 93 125 us per step at 32 x 8, H = 14, against 140
     // at H = 8; 200^3 MRT 592 us at 64 x 4, H = 40, against 816 with
     // registers). Reach-2 stencils in FP64 leave one of its blocks per CU and
     // stay on registers (96^3 E8: 78 us against 131), as does the dense MRT

@@ -106,8 +106,8 @@ struct Impl {
       const int nty = S::D == 3 ? (g.L1 + TY - 1) / TY : 1;
       const int Lm = S::D == 3 ? g.L2 : g.L1;
       // 3D: a march for these tiles, not for the tile that the step without
-      // walls runs (77 x 68 x 278: 163 us per step, 220 with the H of 32 x 8;
-      // 96^3 86 and 111)
+      // walls runs (77 x 68 x 278: 150 us per step, 214 with the H of 32 x 8;
+      // 96^3 83 and 107)
       const int H = S::D == 3 && s->auto_launch
                         ? march_planes((int64_t)ntx * nty, Lm, ES::R)
                         : std::min(s->H, Lm);
