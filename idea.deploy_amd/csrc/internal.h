@@ -103,8 +103,14 @@ struct SimOps {
                       const double* coeffs);
 };
 
-const SimOps* get_ops_d2q9_f64(int estencil, int coll);
-const SimOps* get_ops_d2q9_f32(int estencil, int coll);
+// One unit per velocity set, stencil and precision: a simulation's first launch
+// loads the whole unit that the kernel is in.
+const SimOps* get_ops_d2q9_e4_f64(int coll);
+const SimOps* get_ops_d2q9_e4_f32(int coll);
+const SimOps* get_ops_d2q9_e6_f64(int coll);
+const SimOps* get_ops_d2q9_e6_f32(int coll);
+const SimOps* get_ops_d2q9_e8_f64(int coll);
+const SimOps* get_ops_d2q9_e8_f32(int coll);
 const SimOps* get_ops_d3q19_e4_f64(int coll);
 const SimOps* get_ops_d3q19_e4_f32(int coll);
 const SimOps* get_ops_d3q19_e6_f64(int coll);

@@ -374,14 +374,14 @@ int idmx_sc_create(idmx_ctx_t c, const idmx_sc_desc* d, idmx_sc_t* out) {
   s->geo.V = V;
   s->pop_elem = d->precision == IDMX_PREC_F64 ? 8 : 4;
   const bool f64 = d->precision == IDMX_PREC_F64;
-  if (D == 2)
-    s->ops = f64 ? get_ops_d2q9_f64(d->estencil, s->coll) : get_ops_d2q9_f32(d->estencil, s->coll);
-  else if (d->estencil == IDMX_E4)
-    s->ops = f64 ? get_ops_d3q19_e4_f64(s->coll) : get_ops_d3q19_e4_f32(s->coll);
-  else if (d->estencil == IDMX_E6)
-    s->ops = f64 ? get_ops_d3q19_e6_f64(s->coll) : get_ops_d3q19_e6_f32(s->coll);
-  else
-    s->ops = f64 ? get_ops_d3q19_e8_f64(s->coll) : get_ops_d3q19_e8_f32(s->coll);
+  const SimOps* (*const units[2][3][2])(int) = {
+      {{get_ops_d2q9_e4_f32, get_ops_d2q9_e4_f64},
+       {get_ops_d2q9_e6_f32, get_ops_d2q9_e6_f64},
+       {get_ops_d2q9_e8_f32, get_ops_d2q9_e8_f64}},
+      {{get_ops_d3q19_e4_f32, get_ops_d3q19_e4_f64},
+       {get_ops_d3q19_e6_f32, get_ops_d3q19_e6_f64},
+       {get_ops_d3q19_e8_f32, get_ops_d3q19_e8_f64}}};
+  s->ops = units[D == 3][d->estencil / 2 - 2][f64](s->coll);
   if (!s->ops) {
     delete s;
     set_error("idmx_sc_create: unsupported combination");

@@ -1,5 +1,5 @@
 // sc_impl.h -- host-side launch logic for one (velocity set, E-stencil,
-// precision, collision) combination. Included by sc_d2q9.hip / sc_d3q19.hip,
+// precision, collision) combination. Included by the sc_d*_e*.hip units,
 // which instantiate the combinations of their velocity set.
 #pragma once
 #include <algorithm>

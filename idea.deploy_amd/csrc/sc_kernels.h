@@ -620,8 +620,12 @@ __device__ inline void local_store(T* __restrict__ dst, const Geom& geo, int x, 
 // Conversion between streamed populations and the pull form:
 // dir = +1: dst_q(x) = src_q(x + c_q) (streamed -> pull form),
 // dir = -1: dst_q(x) = src_q(x - c_q) (pull form -> streamed).
+//
+// This and the other kernels that have no stencil as a parameter are static:
+// otherwise all units share one of them, and a simulation's first use of it
+// loads the code of another unit as well.
 template <class S, class T>
-__global__ void __launch_bounds__(256)
+static __global__ void __launch_bounds__(256)
 k_restream(const T* __restrict__ src, T* __restrict__ dst, Geom geo, int dir) {
   for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < geo.V;
        g += (int64_t)gridDim.x * blockDim.x) {
@@ -1399,7 +1403,7 @@ __device__ inline void push_store_walls(T* __restrict__ dst, const Geom& geo,
 // PROG: psi from the compiled psi_code program (a separate instantiation, so
 // that the closed forms keep their registers and occupancy).
 template <class S, class T, bool SHIFT, bool PROG = false>
-__global__ void __launch_bounds__(256)
+static __global__ void __launch_bounds__(256)
 k_density_psi(const T* __restrict__ pop, Geom geo, Phys<T> P,
               double* __restrict__ n, double* __restrict__ psi,
               const uint8_t* __restrict__ walls) {
@@ -1440,7 +1444,7 @@ __device__ inline void site_xyz(const Geom& geo, int64_t g, int& x, int& y, int&
 // flags: recomputed at every run, so flags changed between runs are seen.
 // Writes 1 to *other when a flag is neither 0 nor 1.
 template <class S>
-__global__ void __launch_bounds__(256)
+static __global__ void __launch_bounds__(256)
 k_wall_mask(const uint8_t* __restrict__ walls, Geom geo, uint64_t* __restrict__ mask,
             uint32_t* __restrict__ other) {
   for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < geo.V;
@@ -1529,7 +1533,7 @@ k_velocity(const T* __restrict__ pop, const double* __restrict__ n_in,
 
 // K_InitPopulations: f = f_eq(n, u) (idpy/LBM/LBM.py:1700-1743).
 template <class S, class T, bool SHIFT>
-__global__ void __launch_bounds__(256)
+static __global__ void __launch_bounds__(256)
 k_init_pop(T* __restrict__ pop, const double* __restrict__ n,
            const double* __restrict__ u, Geom geo, double rho0) {
   for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < geo.V;
@@ -1561,7 +1565,7 @@ struct EqTab {
 };
 
 template <class S, class T, bool SHIFT>
-__global__ void __launch_bounds__(256)
+static __global__ void __launch_bounds__(256)
 k_init_pop_tab(T* __restrict__ pop, const double* __restrict__ n, const double* __restrict__ u,
                Geom geo, double rho0, EqTab<NBasis<S::D>::value * S::Q> tab) {
   constexpr int NB = NBasis<S::D>::value;
@@ -1585,7 +1589,7 @@ k_init_pop_tab(T* __restrict__ pop, const double* __restrict__ n, const double* 
 
 // Device population layout <-> float64 SoA (adds / removes the shift).
 template <class S, class T, bool SHIFT>
-__global__ void __launch_bounds__(256)
+static __global__ void __launch_bounds__(256)
 k_pop_to_f64(const T* __restrict__ pop, double* __restrict__ dst, Geom geo, double rho0) {
   for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < geo.V;
        g += (int64_t)gridDim.x * blockDim.x) {
@@ -1599,7 +1603,7 @@ k_pop_to_f64(const T* __restrict__ pop, double* __restrict__ dst, Geom geo, doub
 }
 
 template <class S, class T, bool SHIFT>
-__global__ void __launch_bounds__(256)
+static __global__ void __launch_bounds__(256)
 k_pop_from_f64(T* __restrict__ pop, const double* __restrict__ src, Geom geo, double rho0) {
   for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < geo.V;
        g += (int64_t)gridDim.x * blockDim.x) {
@@ -1642,7 +1646,7 @@ __device__ inline double block_reduce(double v) {
 // Per-block mass and momentum partials of a population buffer:
 // out[b*4 + 0] = sum n, out[b*4 + 1 + d] = sum j_d.
 template <class S, class T, bool SHIFT>
-__global__ void __launch_bounds__(256)
+static __global__ void __launch_bounds__(256)
 k_mass_mom_partial(const T* __restrict__ pop, Geom geo, double rho0,
                    double* __restrict__ out) {
   double m = 0, jx = 0, jy = 0, jz = 0;

@@ -35,7 +35,9 @@ FLAGS = ['-std=c++17', '-O3', '-fPIC', '--offload-arch=' + ARCH,
 # the same step in another launch shape.
 NOFMA = ['-ffp-contract=off']
 INEXPR = ['-ffp-contract=on']
-SOURCES = [('runtime.hip', NOFMA), ('sc_d2q9.hip', NOFMA), ('sc_d2q9_f32.hip', INEXPR),
+SOURCES = [('runtime.hip', NOFMA), ('sc_d2q9_e4.hip', NOFMA), ('sc_d2q9_e4_f32.hip', INEXPR),
+           ('sc_d2q9_e6.hip', NOFMA), ('sc_d2q9_e6_f32.hip', INEXPR),
+           ('sc_d2q9_e8.hip', NOFMA), ('sc_d2q9_e8_f32.hip', INEXPR),
            ('sc_d3q19_e4.hip', NOFMA), ('sc_d3q19_e4_f32.hip', INEXPR),
            ('sc_d3q19_e6.hip', NOFMA), ('sc_d3q19_e6_f32.hip', INEXPR),
            ('sc_d3q19_e8.hip', NOFMA), ('sc_d3q19_e8_f32.hip', INEXPR),
