@@ -111,12 +111,15 @@ def run_gpu(name, steps, warmup, tune=True, launch=None, two_pass=False):
     m1, _ = eng.mass_momentum(pop)
     launch = eng.get_launch()
     itemsize = 8 if w['prec'] == 'fp64' else 4
-    B_alg = 2 * eng.Q * itemsize
+    # a pass over the populations reads and writes each of them once; large 2D
+    # lattices take two steps per pass on variant 10
+    per_pass = 2 if eng.D == 2 and launch[3] == 10 and not two_pass else 1
+    B_alg = 2 * eng.Q * itemsize // per_pass
     res = {
         'V': V, 'Q': eng.Q, 'wall_s': wall, 'event_ms': ev_ms,
         'mlups': V * steps / wall / 1e6,
         'kernel_ms': ev_ms / steps,
-        'B_alg': B_alg,
+        'B_alg': B_alg, 'steps_per_pass': per_pass,
         'mass_rel_drift': abs(m1 - m0) / m0,
         'launch': {'tile_x': launch[0], 'tile_y': launch[1], 'planes_per_block': launch[2],
                    'variant': launch[3], 'variant_name': VARIANTS.get(launch[3], '?')},
@@ -603,7 +606,9 @@ def tune_report(names):
         B = 2 * eng.Q * (8 if w['prec'] == 'fp64' else 4)
         print('%s best %s' % (name, best), flush=True)
         for k, ms in sorted(tim.items(), key=lambda kv: kv[1]):
-            print('  %-16s %.4f ms  %.1f%%' % (k, ms, 100 * B * eng.V / (ms / 1e3) / 8e12),
+            per_pass = 2 if eng.D == 2 and k.endswith(',10') else 1  # steps (run_gpu)
+            print('  %-16s %.4f ms  %.1f%%'
+                  % (k, ms, 100 * B / per_pass * eng.V / (ms / 1e3) / 8e12),
                   flush=True)
         eng.close()
     t.End()
@@ -770,7 +775,8 @@ def main():
         ax = rx['B_alg'] * rx['V'] / (rx['kernel_ms'] / 1e3) / 1e9
         tx, tlx = traffic_from_profiles(x)
         extra[x] = {'mlups': round(rx['mlups'], 1), 'hbm_frac': round(ax / PEAK_HBM_GBS, 4),
-                    'achieved_GBs': round(ax, 1), 'kernel_ms': round(rx['kernel_ms'], 4),
+                    'achieved_GBs': round(ax, 1), 'bytes_per_site': rx['B_alg'],
+                    'steps_per_pass': rx['steps_per_pass'], 'kernel_ms': round(rx['kernel_ms'], 4),
                     'mass_rel_drift': rx['mass_rel_drift'], 'traffic': tx,
                     'traffic_launch': tlx,
                     'launch': [rx['launch'][k] for k in ('tile_x', 'tile_y',
