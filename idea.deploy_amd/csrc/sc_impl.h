@@ -832,11 +832,12 @@ struct Impl {
 
 // Tables over the collision for one (S, ES), FP64 and FP32-shifted. The two
 // precisions are instantiated in separate translation units: the FP64 ones
-// are compiled without floating-point contraction (no fused multiply-add),
-// which is how the reference's CTypes backend computes, so that the FP64
-// trajectory stays within 1e-13 of it over 10^4 steps; with contraction the
-// two drift apart by 2e-11 over the same run. The FP32-shifted step keeps
-// contraction within expressions (its accuracy is set by FP32 storage).
+// are compiled without floating-point contraction (no fused multiply-add), as
+// the reference's CTypes backend is: the 128^2 droplet stays within 1.4e-13
+// of it over 10^4 steps, although collide() adds its terms up in another
+// order; with contraction the two drift apart by 2.1e-11 over the same run.
+// The FP32-shifted step keeps contraction within expressions (its accuracy is
+// set by FP32 storage).
 // coll: 0 BGK, 1 MRT with dense tables, 2 MRT with a diagonal S, 3 BGK with
 // the Shan-Chen forcing, 4 BGK followed by the isotropy filter (D2Q9 and
 // FP64 only; 3 and 4 on one fixed fused launch or the two-pass step).

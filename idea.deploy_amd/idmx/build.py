@@ -26,9 +26,11 @@ FLAGS = ['-std=c++17', '-O3', '-fPIC', '--offload-arch=' + ARCH,
 
 # (source, extra flags). The FP64 lattice code (and the batch and runtime
 # units, whose FP64 results must agree with it bit for bit) is compiled
-# without floating-point contraction, as the reference's CTypes backend
-# computes: with fused multiply-adds the FP64 trajectory drifts from it by
-# 2e-11 over 10^4 steps, without by 1e-13. The FP32-shifted lattice units
+# without floating-point contraction, as the reference's CTypes backend is.
+# The collision's terms are added up in another order than there (opposite
+# velocities share theirs), so the two round differently at every step: the
+# populations of the 128^2 droplet differ by 1.4e-13 after 10^4 steps, with
+# fused multiply-adds by 2.1e-11. The FP32-shifted lattice units
 # (single-domain and batched) contract within an expression only: across
 # expressions (hipcc's default, which the network kernels keep) the choice of
 # fused operations differs from kernel to kernel, and with it the last bits of
