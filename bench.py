@@ -538,7 +538,7 @@ def run_batch_step_study(n_points, Lmax, steps, launch=None):
     2 * steps and a run of `steps` (each run twice, the second timed: the
     first captures its graph; the difference cancels the pull form's
     conversions). Algorithmic bytes 144 per site (nine FP64 populations read
-    once and written once)."""
+    once and written once), 72 with two steps per pass (kinds 4 and 5)."""
     from idmx import configs, sweep, tune
     from idmx.IdpyCode import Tenet
     tenet = Tenet(0)
@@ -555,11 +555,12 @@ def run_batch_step_study(n_points, Lmax, steps, launch=None):
     t_b = b.run(2 * steps)
     ms = (t_b - t_a) / steps
     sites = int(sum(p.L * p.L for p in pts))
-    gbs = 144 * sites / (ms / 1e3) / 1e9
+    nbytes = 72 if launch[0] in (4, 5) else 144
+    gbs = nbytes * sites / (ms / 1e3) / 1e9
     out = {'n_points': n_points, 'L': [64, Lmax], 'sites': sites, 'launch': list(launch),
            'work_items': b.get_launch()[4], 'steps_timed': steps, 'ms_per_step': ms,
            'mlups': sites / (ms / 1e3) / 1e6, 'achieved_GBs': gbs,
-           'hbm_frac': gbs / PEAK_HBM_GBS, 'bytes_per_site': 144}
+           'hbm_frac': gbs / PEAK_HBM_GBS, 'bytes_per_site': nbytes}
     b.close()
     tenet.End()
     return out
